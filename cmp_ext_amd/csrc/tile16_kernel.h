@@ -12,18 +12,20 @@
 //     grain lets a 256 x 224 tile (the MLP shape) use the same grid as 256 x 256.
 //   * Two waves per SIMD: the 256-row tiles run 8 waves (4 x 2, at most 256
 //     VGPRs each) in one workgroup per CU, the 128 x 128 tile 4 waves (2 x 2) in
-//     two workgroups per CU.  One wave's matrix products then run while the other
-//     waits on LDS reads or on the issue of its LDS-DMA loads; measured on
+//     two workgroups per CU -- or alone on its CU with a deeper ring, when there are
+//     no more workgroups than CUs (deep_ring in tile_inst.h).  One wave's matrix products
+//     then run while the other waits on LDS reads or on the issue of its LDS-DMA loads; measured on
 //     MI355X, 8 waves beat 4 waves of twice the block (fewer fragment bytes per
 //     MFMA, one wave per SIMD) by ~9 % in loop cycles and halve the epilogue.
 //   * K steps of BK = 64 go global -> LDS by buffer_load_dwordx4 ... lds (LDS
-//     DMA: no registers, no ds_write) into a two-stage ring.  A step is two
+//     DMA: no registers, no ds_write) into a ring of two slots (or four).  A step is two
 //     sub-steps of 32 k.  All reads of a step's slot are issued by the end of its
 //     first sub-step (they fetch the second sub-step's fragments), so one barrier
 //     between the two sub-steps both frees slot t and certifies step t+1; the
 //     second sub-step then reads step t+1's first fragments and issues all of
 //     step t+2's DMA into slot t, which has a sub-step and a half to land before
-//     the next barrier.
+//     the next barrier (four slots: step t+4's, half of it in step t+1's first
+//     sub-step, with three steps to land).
 //   * A (and B given as [N,K]) are K-contiguous: LDS rows of 128 bytes in the
 //     lds_off128 layout, one ds_read_b128 per 16 x 32 fragment, conflict free.
 //   * B given as [K,N] stays [k][n] in LDS (rows padded to a multiple of 256
@@ -58,7 +60,8 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-template <int BM, int BN, bool KN, int WM, int WN>
+// NS: ring slots, one K step of BK each.
+template <int BM, int BN, bool KN, int WM, int WN, int NS = 2>
 struct Tile16Shape {
   static constexpr int BK = 64;
   static constexpr int ROW = BK * 2;  // bytes per LDS row of a K-contiguous operand
@@ -68,18 +71,20 @@ struct Tile16Shape {
   static constexpr int A_BYTES = BM * ROW;
   static constexpr int B_PITCH = KN ? (BN * 2 + 255) / 256 * 256 : ROW;  // bytes per LDS row of B
   static constexpr int B_BYTES = KN ? BK * B_PITCH : (BN + 63) / 64 * 64 * ROW;  // rows >= BN are OOB
-  // LDS: the two ring slots of A, then the two of B, so that a fragment read of either
-  // slot is a fixed base register plus an immediate offset below 64 KiB
-  static constexpr int B_REGION = 2 * A_BYTES;
-  static constexpr int LDS = 2 * (A_BYTES + B_BYTES);
+  // LDS: the ring slots of A, then those of B, so that a fragment read of any slot is a
+  // fixed base register plus an immediate offset below 64 KiB
+  static constexpr int B_REGION = NS * A_BYTES;
+  static constexpr int LDS = NS * (A_BYTES + B_BYTES);
   static constexpr int A_DMA = A_BYTES / 1024 / NW;  // 1 KB LDS-DMA loads per wave per step
   static constexpr int B_DMA = B_BYTES / 1024 / NW;
   static constexpr int DMA = A_DMA + B_DMA;
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "16-row/column blocks");
   static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0, "whole DMA loads per wave");
   static_assert(LDS <= 160 * 1024, "LDS budget");
-  static_assert(DMA <= 63, "vmcnt range");
-  static_assert(A_BYTES + 14 * 2048 <= 65535 && B_BYTES + 36 * B_PITCH <= 65535, "immediate LDS offsets");
+  static_assert(NS >= 2 && (NS - 1) * DMA <= 63, "vmcnt range");
+  static_assert((NS - 1) * A_BYTES + (FM - 1) * 2048 <= 65535 &&
+                    (NS - 1) * B_BYTES + (KN ? 36 * B_PITCH : (FN - 1) * 2048) <= 65535,
+                "immediate LDS offsets");
 };
 
 // BIAS: 0 none, 1 per column of C (Linear), 2 per row (conv 1x1).  A kernel per
@@ -90,9 +95,9 @@ struct Tile16Shape {
 // KCHECK: K (every split's K range) is not a multiple of 64, so the loads compare
 // each piece's k with K; otherwise they load whole steps unchecked.
 template <typename T, bool KN, int BM, int BN, int WM, int WN, int BIAS, int MINB, bool SPLITK = false,
-          bool KCHECK = false>
+          bool KCHECK = false, int NS = 2>
 __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const GemmParams p) {
-  using S = Tile16Shape<BM, BN, KN, WM, WN>;
+  using S = Tile16Shape<BM, BN, KN, WM, WN, NS>;
   constexpr int FM = S::FM, FN = S::FN;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[S::LDS];
 
@@ -142,7 +147,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const G
       b_kx[i] = 8 * chunk;
     }
   }
-  // LDS-DMA load d (A pieces first, then B) of K step kt into ring slot kt % 2.  A (and B
+  // LDS-DMA load d (A pieces first, then B) of K step kt into ring slot kt % NS.  A (and B
   // as [N,K]) keep one descriptor at the tile base and advance along K through the SGPR
   // offset; B as [K,N] gets a descriptor per step.  The destination goes through M0
   // (one s_add per piece from a per-wave base).  With CHECK each piece's k is compared
@@ -233,13 +238,13 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const G
     }
   };
   // One 32-k sub-step of MFMAs on fragment buffer BUF; MFMA slot x also issues read
-  // r * X / RD == x of sub-step RS of ring slot RSLOT into the other buffer and, for
-  // DMA mode 1 (full step) or 2 (the step holding K's end), DMA piece d * X / DMA == x of
-  // step dkt into ring slot DSLOT.
+  // r * X / RD == x of sub-step RS of ring slot RSLOT into the other buffer and its share
+  // of DMA pieces D0 .. D1-1 of step dkt into ring slot DSLOT.
   constexpr int X = FM * FN;
-  auto substep = [&](auto bufc, auto rslotc, int rs, auto dmac, int dkt, auto dslotc) {
+  using Check = std::integral_constant<bool, KCHECK>;
+  auto substep = [&](auto bufc, auto rslotc, int rs, auto d0c, auto d1c, int dkt, auto dslotc) {
     constexpr int buf = decltype(bufc)::value;
-    constexpr int dma = decltype(dmac)::value;
+    constexpr int d0 = decltype(d0c)::value, nd = decltype(d1c)::value - d0;
     static_for<X>([&](auto xc) {
       constexpr int x = decltype(xc)::value;
       constexpr int i = x / FN, j = x % FN;
@@ -247,41 +252,56 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const G
       static_for<RD>([&](auto rc) {
         if constexpr (decltype(rc)::value * X / RD == x) read_one(rslotc, rs, buf ^ 1, rc);
       });
-      if constexpr (dma != 0) {
-        static_for<S::DMA>([&](auto dc) {
-          if constexpr (decltype(dc)::value * X / S::DMA == x)
-            dma_piece(dkt, dslotc, dc, std::integral_constant<bool, dma == 2>{});
-        });
-      }
+      static_for<nd>([&](auto dc) {
+        if constexpr (decltype(dc)::value * X / nd == x)
+          dma_piece(dkt, dslotc, std::integral_constant<int, d0 + decltype(dc)::value>{}, Check{});
+      });
       __builtin_amdgcn_sched_barrier(0);  // keep the slots in this order
     });
   };
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
+  using DH = std::integral_constant<int, NS == 2 ? 0 : S::DMA / 2>;  // pieces left for the next step's first half
+  using DL = std::integral_constant<int, S::DMA - DH::value>;
+  using DA = std::integral_constant<int, S::DMA>;
   // K step kt from ring slot SLOT: the second half's fragments are read during the
   // first sub-step; one barrier certifies that every read of the slot is done and
-  // that step kt+1 (the other slot) has landed; the second sub-step reads step
-  // kt+1's first fragments and loads step kt+2 into this slot (DMA mode as above).
-  auto step = [&](int kt, auto slotc, auto dmac) {
-    using Other = std::integral_constant<int, 1 - decltype(slotc)::value>;
-    substep(B0{}, slotc, 1, B0{}, 0, slotc);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
-    substep(B1{}, Other{}, 0, dmac, kt + 2, slotc);
+  // that step kt+1 (the next slot) has landed (steps kt+2 .. kt+NS-1 may be in flight);
+  // the second sub-step reads step kt+1's first fragments and loads step kt+NS into
+  // this slot.  A deeper ring leaves the last DH pieces of that load to the next step's
+  // first sub-step (they have two more steps to land), so that the loads' issue (a CU
+  // takes 64 bytes per cycle) is spread over the whole step.
+  auto step = [&](int kt, auto slotc) {
+    using Next = std::integral_constant<int, (decltype(slotc)::value + 1) % NS>;
+    using Prev = std::integral_constant<int, (decltype(slotc)::value + NS - 1) % NS>;
+    substep(B0{}, slotc, 1, DL{}, DA{}, kt + NS - 1, Prev{});
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((NS - 2) * S::DMA) : "memory");
+    substep(B1{}, Next{}, 0, B0{}, DL{}, kt + NS, slotc);
   };
 
   const int nk = (K + S::BK - 1) / S::BK;
   if (nk > 0) {
-    using Mode = std::integral_constant<int, KCHECK ? 2 : 1>;  // checked or whole-step loads
-    using Check = std::integral_constant<bool, KCHECK>;
-    static_for<S::DMA>([&](auto dc) { dma_piece(0, B0{}, dc, Check{}); });
-    static_for<S::DMA>([&](auto dc) { dma_piece(1, B1{}, dc, Check{}); });  // zeros if nk == 1
+    // steps 0 and 1, then (a deeper ring) the rest of the ring once step 0 has landed and its
+    // first fragments are on their way, so that those loads' issue does not delay them; steps
+    // past the end load zeros
+    auto fill = [&](auto sc) {
+      static_for<S::DMA>([&](auto dc) {
+        if constexpr (NS == 2 || decltype(sc)::value < NS - 1 || decltype(dc)::value < DL::value)
+          dma_piece(decltype(sc)::value, sc, dc, Check{});
+      });
+    };
+    fill(B0{});
+    fill(B1{});
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(S::DMA) : "memory");  // step 0 landed
     static_for<RD>([&](auto rc) { read_one(B0{}, 0, 0, rc); });
-    // pairs of steps, ring slots 0 and 1 (two copies of the step's code: the slot offsets
-    // are immediates)
-    for (int kt = 0; kt < nk; kt += 2) {
-      step(kt, B0{}, Mode{});
-      if (kt + 1 < nk) step(kt + 1, B1{}, Mode{});
+    static_for<NS - 2>([&](auto sc) { fill(std::integral_constant<int, decltype(sc)::value + 2>{}); });
+    // NS steps, one per ring slot (NS copies of the step's code: the slot offsets are
+    // immediates)
+    for (int kt = 0; kt < nk; kt += NS) {
+      static_for<NS>([&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        if (s == 0 || kt + s < nk) step(kt + s, sc);
+      });
     }
     asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // no LDS DMA may outlive the workgroup
   }
@@ -401,20 +421,20 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const G
   });
 }
 
-// Launches gemm_tile16_kernel (WM x WN waves, MINB workgroups per CU) with the
-// bias mode and the K split the arguments ask for.
-template <typename T, bool KN, int BM, int BN, int WM, int WN, int MINB, bool KCHECK>
+// Launches gemm_tile16_kernel (WM x WN waves, MINB workgroups per CU, NS ring slots) with
+// the bias mode and the K split the arguments ask for.
+template <typename T, bool KN, int BM, int BN, int WM, int WN, int MINB, bool KCHECK, int NS = 2>
 hipError_t launch_tile16_k(const GemmParams& p, dim3 grid, hipStream_t s) {
   const dim3 block(64 * WM * WN);
   if constexpr (BM >= 128) {
     if (p.splits > 1)  // fp32 partials; the bias comes with the reduction
-      return launch_kernel((gemm_tile16_kernel<T, KN, BM, BN, WM, WN, 0, MINB, true, KCHECK>), grid, block, 0, s, p);
+      return launch_kernel((gemm_tile16_kernel<T, KN, BM, BN, WM, WN, 0, MINB, true, KCHECK, NS>), grid, block, 0, s, p);
   }
   if (p.bias == nullptr)
-    return launch_kernel((gemm_tile16_kernel<T, KN, BM, BN, WM, WN, 0, MINB, false, KCHECK>), grid, block, 0, s, p);
+    return launch_kernel((gemm_tile16_kernel<T, KN, BM, BN, WM, WN, 0, MINB, false, KCHECK, NS>), grid, block, 0, s, p);
   if (p.bias_row)
-    return launch_kernel((gemm_tile16_kernel<T, KN, BM, BN, WM, WN, 2, MINB, false, KCHECK>), grid, block, 0, s, p);
-  return launch_kernel((gemm_tile16_kernel<T, KN, BM, BN, WM, WN, 1, MINB, false, KCHECK>), grid, block, 0, s, p);
+    return launch_kernel((gemm_tile16_kernel<T, KN, BM, BN, WM, WN, 2, MINB, false, KCHECK, NS>), grid, block, 0, s, p);
+  return launch_kernel((gemm_tile16_kernel<T, KN, BM, BN, WM, WN, 1, MINB, false, KCHECK, NS>), grid, block, 0, s, p);
 }
 
 }  // namespace cmpext3
