@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "gemm_params.h"
 
@@ -18,6 +19,17 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+// f(std::integral_constant<int, I>) for I = 0 .. N-1, fully unrolled (register
+// arrays indexed by I stay in registers).
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
 
 // Offset that is always outside a buffer resource whose num_records is
 // kBufRecords: a buffer load with it returns zeros and touches no memory.

@@ -138,7 +138,7 @@ namespace {
 struct Override {
   int kernel = -1;
   int splits = 1;
-  int strip = 0;  // rows of A (tall: 32 or 64) or of W (skinny_nk: 16, 32 or 64) per workgroup; 0: the selector's
+  int strip = 0;  // rows of A (tall: 32 or 64) or of W (skinny_nk: 16 to 128) per workgroup; 0: the selector's
 };
 
 Override read_override() {
@@ -157,7 +157,7 @@ Override read_override() {
       if (v >= 1 && v <= 16) o.splits = v;
     } else if (strncmp(tok, "strip=", 6) == 0) {
       const int v = atoi(tok + 6);
-      if (v == 16 || v == 32 || v == 64) o.strip = v;
+      if (v > 0 && v <= 128 && v % 16 == 0) o.strip = v;
     }
   }
   return o;
@@ -188,14 +188,41 @@ void split_strips(const Request& r, int64_t splits, Plan* q) {
   }
 }
 
-// skinny_nk (M <= 64, B as [N, K]): strips of W rows over all of K, or over K ranges of
-// `splits` (fp32 partials in the workspace, N % 4 == 0; a split that does not fit the
-// workspace is dropped).  16-row strips when 32-row ones would leave CUs idle.  With more
-// than 16 rows of A every workgroup re-reads all of A from L2 (for 64 x 4096: twice W's
-// bytes over 448 strips of a 14336-row W), so 64-row strips there once they still give
-// >= 192 workgroups (MI355X, x[M, 4096] W[14336, 4096]^T: M = 32 27.7 -> 23.9 us, 48 30.2
-// -> 26.8, 64 34.1 -> 29.3; x[64, 8192] W[14336, 8192]^T 56.8 -> 51.6; x[64, 8192]
-// W[28672, 8192]^T 111 either way).
+// Rows of W per workgroup of skinny_nk (M <= 64, B as [N, K]; mb 16-row blocks of A), for
+// N rows of W in each of `batch` entries.  A CU runs one of these workgroups at a time
+// (two of the 32-row ones with one block of A) and takes in bytes at a rate that hardly
+// depends on the strip, so the time goes with the rounds of 256 workgroups times the rows
+// that one streams, its own of W and all of A's: the height with the least of that, 16 to
+// 128.  Narrow strips in 1.3 or 1.8 rounds reread A in each of them and leave CUs idle in
+// the last (MI355X, bf16, W from HBM, against 16, 32 or 64 rows as CUs and blocks of A
+// had it before: x[64, 4096] W[11008, 4096]^T 48 rows 32.8 -> 24.2 us, x[64, 5120]
+// W[20480, 5120]^T 80 rows 63.5 -> 40.6, x[64, 4096] W[24576, 4096]^T 96 rows 55.6 ->
+// 45.7, x[64, 4096] W[28672, 4096]^T 112 rows 57.5 -> 51.7, x[32, 4096] W[6144, 4096]^T
+// 32 rows 15.9 -> 11.8; x[64, 4096] W[14336, 4096]^T 64 rows as before, 80 rows 30.9
+// against 29.3).  One block of A: 16, 32 or 48 rows in one round, else 32-row strips two
+// to a CU (x[16, 4096] W[11008, 4096]^T 48 rows 19.9 -> 17.3, W[6144, 4096]^T 32 rows
+// 13.4 -> 10.8; past 48 x 256 rows two of 32 per CU stay ahead: W[14336, 4096]^T 21.3
+// against 22.9 with 64 rows, W[28672, 4096]^T 39.9 against 43.1).
+int skinny_nk_strip(int64_t N, int64_t batch, int mb) {
+  if (mb == 1) {
+    for (int rows = 16; rows <= 48; rows += 16)
+      if (cdiv(N, rows) * batch <= kNumCUs) return rows;
+    return 32;
+  }
+  int best = 16;
+  int64_t least = 0;
+  for (int rows = 16; rows <= 128; rows += 16) {
+    const int64_t streamed = cdiv(cdiv(N, rows) * batch, kNumCUs) * (rows + 16 * mb);
+    if (rows == 16 || streamed < least) {
+      best = rows;
+      least = streamed;
+    }
+  }
+  return best;
+}
+
+// skinny_nk: strips of W rows over all of K, or over K ranges of `splits` (fp32 partials in
+// the workspace, N % 4 == 0; a split that does not fit the workspace is dropped).
 Plan skinny_nk_plan(const Request& r, int64_t splits, int group_m) {
   Plan q{};
   q.kernel = kSkinnyNK;
@@ -205,8 +232,7 @@ Plan skinny_nk_plan(const Request& r, int64_t splits, int group_m) {
   q.mb = (int)std::max<int64_t>(1, cdiv(r.M, 16));
   q.bm = 16 * q.mb;
   const int64_t chunk = std::min<int64_t>(r.batch, 65535);
-  q.bn = cdiv(r.N, 32) * chunk >= kNumCUs ? 32 : 16;
-  if (q.mb >= 2 && cdiv(r.N, 64) * chunk >= 192) q.bn = 64;
+  q.bn = skinny_nk_strip(r.N, chunk, q.mb);
   split_strips(r, splits, &q);
   return q;
 }
@@ -272,7 +298,7 @@ void override16(const Request& r, bool fast, bool stream_ok, bool tall_ok, bool 
     case kSkinnyNK:
       if (!skinny_nk_ok) return;
       q = skinny_nk_plan(r, o.splits, p->group_m);
-      if (o.strip) q.bn = o.strip;
+      if (o.strip && (q.mb > 1 || o.strip <= 64)) q.bn = o.strip;
       break;
     case kTall:
       // strips of 32 or 64 rows of A only (0: 64); a 16-row strip is not built for it

@@ -27,9 +27,9 @@ namespace {
 template <typename T, int SW, bool NT>
 hipError_t launch_nk(int mb, const GemmParams& p, dim3 grid, hipStream_t s) {
   const dim3 block(256);
-  // 1 KiB of each W row per stage for one 16-row block of A, 512 bytes otherwise; 64-row
-  // strips: 512 bytes for one or two blocks, 256 for three or four (the ring keeps >= 3
-  // stages).  32-row strips with one block (more than 256 of them): 512-byte stages in a
+  // 1 KiB of each W row per stage for one 16-row block of A, 512 bytes otherwise; strips of
+  // 48 rows and more: 512 bytes for one or two blocks (up to 64 rows), 256 otherwise (the
+  // ring keeps >= 3 stages).  Strips above 64 rows are for two blocks and more.  32-row strips with one block (more than 256 of them): 512-byte stages in a
   // ring of 3 (72 KiB), so that two workgroups share a CU and all strips run at once
   // instead of in 1.75 rounds (MI355X, x[1, 4096] W[14336, 4096]^T 21.4 -> 19.7 us,
   // x[16, 4096] 23.3 -> 21.4 us, x[1, 8192] W[28672, 8192]^T 76.1 -> 73.3 us; with 16-row
@@ -38,20 +38,33 @@ hipError_t launch_nk(int mb, const GemmParams& p, dim3 grid, hipStream_t s) {
     case 1:
       if constexpr (SW == 32)
         return launch_kernel((gemm_skinny_nk_kernel<T, 1, 32, 256, NT, 3>), grid, block, 0, s, p);
+      else if constexpr (SW <= 64)
+        return launch_kernel((gemm_skinny_nk_kernel<T, 1, SW, SW >= 48 ? 256 : 512, NT>), grid, block, 0, s, p);
       else
-        return launch_kernel((gemm_skinny_nk_kernel<T, 1, SW, SW == 64 ? 256 : 512, NT>), grid, block, 0, s, p);
-    case 2: return launch_kernel((gemm_skinny_nk_kernel<T, 2, SW, 256, NT>), grid, block, 0, s, p);
-    case 3: return launch_kernel((gemm_skinny_nk_kernel<T, 3, SW, SW == 64 ? 128 : 256, NT>), grid, block, 0, s, p);
-    case 4: return launch_kernel((gemm_skinny_nk_kernel<T, 4, SW, SW == 64 ? 128 : 256, NT>), grid, block, 0, s, p);
+        return hipErrorInvalidValue;
+    case 2: return launch_kernel((gemm_skinny_nk_kernel<T, 2, SW, (SW > 64 ? 128 : 256), NT>), grid, block, 0, s, p);
+    case 3: return launch_kernel((gemm_skinny_nk_kernel<T, 3, SW, SW >= 48 ? 128 : 256, NT>), grid, block, 0, s, p);
+    case 4: return launch_kernel((gemm_skinny_nk_kernel<T, 4, SW, SW >= 48 ? 128 : 256, NT>), grid, block, 0, s, p);
     default: return hipErrorInvalidValue;
   }
 }
 template <typename T>
 hipError_t launch_nk(int mb, int strip, const GemmParams& p, dim3 grid, hipStream_t s) {
   const bool nt = stream_once(p.N, p.K, p.stride_b, grid.z);
-  if (strip == 16) return nt ? launch_nk<T, 16, true>(mb, p, grid, s) : launch_nk<T, 16, false>(mb, p, grid, s);
-  if (strip == 64) return nt ? launch_nk<T, 64, true>(mb, p, grid, s) : launch_nk<T, 64, false>(mb, p, grid, s);
-  return nt ? launch_nk<T, 32, true>(mb, p, grid, s) : launch_nk<T, 32, false>(mb, p, grid, s);
+  switch (strip) {
+#define STRIP(SW) \
+  case SW: return nt ? launch_nk<T, SW, true>(mb, p, grid, s) : launch_nk<T, SW, false>(mb, p, grid, s)
+    STRIP(16);
+    STRIP(32);
+    STRIP(48);
+    STRIP(64);
+    STRIP(80);
+    STRIP(96);
+    STRIP(112);
+    STRIP(128);
+#undef STRIP
+    default: return hipErrorInvalidValue;
+  }
 }
 }  // namespace
 

@@ -42,23 +42,9 @@
 //     16-byte stores covering 64 contiguous bytes of each of 16 rows.
 #pragma once
 
-#include <type_traits>
-#include <utility>
-
 #include "device_common.h"
 
 namespace cmpext3 {
-
-// f(std::integral_constant<int, I>) for I = 0 .. N-1, fully unrolled (register
-// arrays indexed by I stay in registers).
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
 
 // NS: ring slots, one K step of BK each.
 template <int BM, int BN, bool KN, int WM, int WN, int NS = 2>
