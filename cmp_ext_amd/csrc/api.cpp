@@ -29,7 +29,7 @@ int align_of(const void* ptr) {
 // The tile kernel for the element type and B layout, with whole-step loads when K
 // (and every split's K range) is a multiple of 64.
 hipError_t launch_tile(int dtype, KernelId id, BLayout lay, const GemmParams& p, dim3 grid, hipStream_t s) {
-  const bool ragged = p.K % 64 != 0 || (p.splits > 1 && p.ksplit % 64 != 0);
+  const bool ragged = p.K % 64 != 0 || (p.splits > 1 && p.ksplit % 64 != 0) || p.b_dword;
   if (dtype == kF16) {
     if (lay == kKN) return ragged ? launch_tile_f16_kn_ragged(id, p, grid, s) : launch_tile_f16_kn_whole(id, p, grid, s);
     return ragged ? launch_tile_f16_nk_ragged(id, p, grid, s) : launch_tile_f16_nk_whole(id, p, grid, s);
@@ -254,6 +254,7 @@ int run(const Prepared& pc, void* workspace, int64_t workspace_bytes, hipStream_
   GemmParams p{};
   p.bias = pc.bias;
   p.bias_row = pc.bias_row;
+  p.b_dword = plan.b_dword;
   p.bias_vec = pc.bias != nullptr && align_of(pc.bias) >= 8;
   p.lda = lda;
   p.ldb = ldb;

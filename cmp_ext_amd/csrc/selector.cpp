@@ -395,9 +395,9 @@ int make_plan_core(const Request& r, Plan* plan) {
                            r.lda % 8 == 0 && r.N % 8 == 0 && r.ldb % 8 == 0 &&
                            (!batched || (r.stride_a % 8 == 0 && r.stride_b % 8 == 0));
     // (the tiled kernels' epilogue stores in 16-, 8- or 2-byte pieces as C's rows allow)
-    const bool fast = r.align >= 16 && r.K % 8 == 0 && r.lda % 8 == 0 && r.ldb % 8 == 0 &&
-                      (r.layout == kNK || r.N % 8 == 0 || r.b_cols_padded) &&
-                      (!batched || (r.stride_a % 8 == 0 && r.stride_b % 8 == 0));
+    const bool fast = r.align >= 16 && r.K % 8 == 0 && r.lda % 8 == 0 && (r.ldb % 8 == 0 || r.b_dword) &&
+                      (r.layout == kNK || r.N % 8 == 0 || r.b_cols_padded || r.b_dword) &&
+                      (!batched || (r.stride_a % 8 == 0 && (r.stride_b % 8 == 0 || r.b_dword)));
     // With M <= 64 the skinny kernels pay off only where the GPU would otherwise
     // starve: once 128-column tiles alone give every CU one (N >= 32768, or a
     // batch of such products, e.g. a 1x1 convolution over many pixels), the tiled
@@ -407,7 +407,7 @@ int make_plan_core(const Request& r, Plan* plan) {
     const bool skinny_tiles_enough = fast && cdiv(r.N, 128) * r.batch >= kNumCUs;
     // what the streaming kernel needs (one A for the batch, C's rows in 16-byte pieces, ...;
     // B as [K,N] or [N,K]; it is chosen below only with enough tiles per workgroup)
-    const bool stream_ok = fast && r.M <= kStreamMaxRows && r.K <= 256 && r.N % 8 == 0 &&
+    const bool stream_ok = fast && !r.b_dword && r.M <= kStreamMaxRows && r.K <= 256 && r.N % 8 == 0 &&
                            r.ldc % 8 == 0 && (!batched || (r.stride_a == 0 && r.stride_c % 8 == 0)) &&
                            (!r.has_bias || r.bias_row) && 128 * r.ldb * 2 <= kIntMax &&
                            128 * r.ldc * 2 <= kIntMax && cdiv(r.N, 128) * r.batch <= kIntMax;
@@ -666,6 +666,24 @@ int make_plan(const Request& r, Plan* plan) {
     b_bytes = cdiv(rows * cols * 2 * ((batched && r.stride_b != 0) ? r.batch : 1), 256) * 256;
   }
   if (a_bytes + b_bytes > r.ws_bytes) return st;
+  // B as [K, N] whose rows are aligned to 4 bytes (an even N or pitch: images of 14 x 14
+  // pixels) needs no copy: a 16-byte LDS-DMA piece only needs a 4-byte aligned source, and
+  // the pieces that cross a row's end bring in columns that are not stored (A's would bring
+  // in wrong k, hence K % 8 == 0).  MI355X, fp16/bf16, copy + aligned tile -> in place:
+  // conv2d [32, 1024, 14, 14] -> 256 25.3 -> 14.7 us, [64, 256, 14, 14] -> 64 15.4 -> 6.8,
+  // 512 x 1002 x 2048 34.6 -> 26.5, 64 x 8190 x 4096 64 -> 42, 4096 x 4090 x 4096 140.7 ->
+  // 134.3, 8192 x 3002 x 1024 95.8 -> 91.6: no shape tried was slower.
+  if (!pad_a && kn && ab >= 4 && r.ldb % 2 == 0 && (!batched || r.stride_b % 2 == 0) && r.K % 8 == 0) {
+    Request d = r;
+    d.b_dword = true;
+    d.align = std::min(aa, ac);
+    Plan p3;
+    if (make_plan_core(d, &p3) == CMPEXT3_OK && p3.kernel != kGeneric16) {
+      p3.b_dword = true;
+      *plan = p3;
+      return CMPEXT3_OK;
+    }
+  }
   q.align_a = pad_a ? 16 : aa;
   q.align_b = pad_b ? 16 : ab;
   q.align = std::min(std::min(q.align_a, q.align_b), ac);
@@ -766,6 +784,7 @@ std::string describe(const Request& r, const Plan& p) {
     s += buf;
   }
   if (p.dma16) s += " dma16";
+  if (p.b_dword) s += " b_dword";
   if (p.pad_a || p.pad_b) {
     snprintf(buf, sizeof buf, " padded=%s%s kp=%lld workspace=%lld", p.pad_a ? "A" : "", p.pad_b ? "B" : "",
              (long long)p.kp, (long long)p.ws_bytes);

@@ -27,6 +27,7 @@ struct Plan {
   int64_t lda_p, ldb_p;                // pitches of the copies
   int64_t stride_a_p, stride_b_p;      // their batch strides (0: one copy shared by the batch)
   int64_t pad_a_bytes, pad_b_bytes;    // workspace bytes of each copy (multiples of 256)
+  bool b_dword;  // 16-bit tile kernels on B as [K, N] whose rows are 4-byte aligned only (no copy of B)
   bool dma16;  // fp32: rows 16-byte aligned, K (and N for B as [K,N]) multiples of 4
   bool forced;  // chosen by the CMPEXT3_GEMM_CONFIG override (no padded copies in its place)
 };
@@ -40,6 +41,7 @@ struct Request {
   int align_a, align_b, align_c;  // the same for A, B and C alone (0: use `align`); the bias
                                   // address never restricts the kernel choice
   bool b_cols_padded;             // B ([K, N]) has zero columns up to a multiple of 8 (planner use)
+  bool b_dword;                   // B ([K, N]) is read in place with 4-byte aligned rows (planner use)
   bool has_bias;
   bool bias_row;  // the bias is one value per row of C (a 1x1 convolution's), not per column
   int64_t batch;

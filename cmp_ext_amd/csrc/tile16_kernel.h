@@ -161,6 +161,15 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const G
       const uint32_t voff = !check || b_kx[i] < K - k0 ? b_off[i] : kBufOOB;
       i32x4 r = KN ? make_rsrc_sgpr(Bbase + (int64_t)(live ? k0 : 0) * ldb) : rsrc_b_nk;
       r[2] = live ? (int)kBufRecords : 0;
+      // B as [K,N] with 4-byte aligned rows: a row's last piece may run into the next row
+      // (columns >= N, which are not stored), the last row's past the operand, so the
+      // descriptor ends where the operand does (the range check is per dword)
+      if constexpr (KN && check) {
+        if (live && p.b_dword) {
+          const int64_t bytes = ((int64_t)(p.K - kbeg - k0 - 1) * ldb + (N - n0)) * (int64_t)sizeof(T);
+          r[2] = bytes < (int64_t)kBufRecords ? (int)bytes : (int)kBufRecords;
+        }
+      }
       dma_load16_m0(r, voff, KN ? 0u : (uint32_t)k0 * (uint32_t)sizeof(T), lds_b, std::integral_constant<uint32_t, dst>{});
     }
   };

@@ -1,0 +1,77 @@
+"""16-bit products whose B is [K, N] with rows aligned to 4 bytes only (an even N or pitch
+that is no multiple of 8: images of 14x14 pixels) are read in place by the tile kernels:
+which calls take that route (CPU), and its results, with NaN after every row and after the
+operand, against the float64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from cmp_ext_amd import cabi
+from oracle import gemm_oracle as O
+
+A, B, C = 0x100000, 0x40000000, 0x80000000  # host addresses: plans only
+
+
+def _plan(M, N, K, lda=None, ldb=None, batch=1, stride_b=None, off_a=0, off_b=0, layout=cabi.B_KN, ws=1 << 40):
+    lda, ldb = lda or K, ldb or (N if layout == cabi.B_KN else K)
+    st, call = cabi.prepare(cabi.F16, layout, A + 2 * off_a, lda, M * lda, B + 2 * off_b, ldb,
+                            stride_b if stride_b is not None else K * ldb, C, N, M * N, None, M, N, K, batch, 0, ws)
+    assert st == cabi.OK
+    return cabi.describe(call)[1]
+
+
+def test_route():
+    rng = np.random.default_rng(7)
+    taken = 0
+    for _ in range(600):
+        M, N, K = int(rng.integers(1, 3000)), int(rng.integers(1, 3000)), int(rng.integers(1, 1500))
+        if rng.random() < 0.7:
+            K = K // 8 * 8 or 8
+        batch, off_b, off_a = int(rng.choice([1, 3])), int(rng.choice([0, 0, 2, 3])), int(rng.choice([0, 0, 0, 4]))
+        ldb = N + int(rng.choice([0, 0, 1, 2, 8]))
+        desc = _plan(M, N, K, ldb=ldb, batch=batch, off_b=off_b, off_a=off_a)
+        aligned_a = K % 8 == 0 and off_a % 8 == 0
+        aligned_b = off_b % 8 == 0 and ldb % 8 == 0 and N % 8 == 0
+        even = off_b % 2 == 0 and ldb % 2 == 0 and (batch == 1 or K * ldb % 2 == 0)
+        expect = aligned_a and even and not aligned_b and M * N * K * batch >= 1 << 24
+        if M <= 64 and N % 8 == 0 and off_b % 8 == 0 and ldb % 8 == 0:
+            expect = False
+        assert ("b_dword" in desc) == expect, (M, N, K, ldb, batch, off_a, off_b, desc)
+        if expect:
+            taken += 1
+            assert "kernel=tile" in desc and "padded" not in desc, desc
+    assert taken > 60
+    assert "generic" in _plan(2048, 60, 2048, ws=0)                # without a workspace: as before
+    assert "padded" in _plan(1000, 1002, 1004)                     # K % 8: A is copied, and B
+    assert "padded=B" in _plan(1000, 1001, 1000)                   # odd rows
+    assert "b_dword" not in _plan(1000, 1002, 1000, layout=cabi.B_NK)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K,gap,off,batch", [
+    (200, 196, 1024, 0, 0, 3), (200, 1002, 512, 0, 0, 1), (257, 1030, 520, 6, 0, 1), (128, 2044, 264, 2, 2, 1),
+    (300, 500, 72, 4, 6, 2), (70, 4098, 320, 0, 0, 1), (513, 130, 4104, 0, 2, 1), (4090, 4090, 128, 0, 0, 1),
+    (64, 70002, 136, 0, 0, 1),
+])
+def test_results(dtype, M, N, K, gap, off, batch):
+    import cmpext3
+
+    dt = {"fp16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    g = torch.Generator().manual_seed(N)
+    a = (torch.randn((batch, M, K), generator=g) * K ** -0.5).to(dt)
+    b = torch.randn((batch, K, N), generator=g).to(dt)
+    ldb = N + gap
+    buf = torch.full((off + batch * K * ldb + 64,), float("nan"), dtype=dt, device="cuda")  # gaps and what follows
+    view = buf[off : off + batch * K * ldb].view(batch, K, ldb)[:, :, :N]
+    view.copy_(b)
+    if batch == 1:
+        fn = cmpext3.fp16_matmul if dtype == "fp16" else cmpext3.bf16_matmul
+        out = fn(a[0].cuda(), view[0])[None]
+    else:
+        out = cmpext3.bmm(a.cuda(), view)
+    desc = cmpext3.last_plan()
+    print(dtype, M, N, K, gap, off, batch, desc, flush=True)
+    assert "b_dword" in desc, desc
+    for i in range(batch):
+        assert O.reference_check(out[i].cpu(), a[i], b[i], dtype) <= O.TOLERANCE[dtype]
