@@ -111,14 +111,16 @@ hipError_t dispatch(const Plan& plan, int dtype, int layout, const GemmParams& p
   }
 }
 
-// A plan's description; for a row split, both launches'.
-std::string describe_rows(const Request& r, const Plan& plan, int64_t m_main, const Plan& tail) {
-  if (m_main <= 0) return describe(r, plan);
+// A plan's description; for a product in two parts, both launches'.
+std::string describe_parts(const Request& r, const Plan& plan, int64_t m_main, int64_t n_main, const Plan& tail) {
+  if (m_main <= 0 && n_main <= 0) return describe(r, plan);
   Request head = r, rest = r;
-  head.M = m_main;
-  rest.M = r.M - m_main;
-  return describe(head, plan) + " rows=" + std::to_string(m_main) + " | rows " + std::to_string(m_main) + ".." +
-         std::to_string(r.M - 1) + ": " + describe(rest, tail);
+  const char* what = m_main > 0 ? "rows" : "cols";
+  const int64_t cut = m_main > 0 ? m_main : n_main, all = m_main > 0 ? r.M : r.N;
+  (m_main > 0 ? head.M : head.N) = cut;
+  (m_main > 0 ? rest.M : rest.N) = all - cut;
+  return describe(head, plan) + " " + what + "=" + std::to_string(cut) + " | " + what + " " + std::to_string(cut) +
+         ".." + std::to_string(all - 1) + ": " + describe(rest, tail);
 }
 
 constexpr int64_t kMaxGridZ = 65535;
@@ -129,8 +131,9 @@ struct Prepared {
   uint64_t magic;
   Request r;
   Plan plan;
-  // rows [0, m_main) run with `plan`, the rest with `tail` (0: one launch for all rows)
-  int64_t m_main;
+  // rows [0, m_main) or columns [0, n_main) run with `plan`, the rest with `tail` (both 0:
+  // one launch for the whole product)
+  int64_t m_main, n_main;
   Plan tail;
   const void* A;
   const void* B;
@@ -177,11 +180,12 @@ int prepare(Prepared* pc, int dtype, int b_layout, const void* A, int64_t lda, i
   p.magic = kCallMagic;
   p.r = r;
   p.plan = plan;
-  RowSplit rs;
-  if (!empty && plan_row_split(r, plan, &rs)) {
-    p.plan = rs.main;
-    p.m_main = rs.m_main;
-    p.tail = rs.tail;
+  TwoPart two;
+  if (!empty && plan_two_parts(r, plan, &two)) {
+    p.plan = two.main;
+    p.m_main = two.m_main;
+    p.n_main = two.n_main;
+    p.tail = two.tail;
   }
   p.A = A;
   p.B = B;
@@ -199,72 +203,39 @@ const Prepared* as_prepared(const cmpext3_gemm_call* call) {
   return pc->magic == kCallMagic ? pc : nullptr;
 }
 
-// Enqueues a prepared call: the zero-padded operand copies it planned, then its
-// kernel(s), batch entries in chunks of at most 65535 grid rows.
-int run(const Prepared& pc, void* workspace, int64_t workspace_bytes, hipStream_t s) {
-  const Plan& plan = pc.plan;
-  if (pc.empty) return CMPEXT3_OK;
-  if (pc.m_main > 0) {  // two launches over the rows, one after the other on the stream
-    const int64_t esz = pc.r.dtype == kF32 ? 4 : 2;
-    Prepared head = pc, rest = pc;
-    head.m_main = rest.m_main = 0;
-    head.r.M = pc.m_main;
-    rest.r.M = pc.r.M - pc.m_main;
-    rest.plan = pc.tail;
-    rest.A = (const char*)pc.A + pc.m_main * pc.r.lda * esz;
-    rest.C = (char*)pc.C + pc.m_main * pc.r.ldc * esz;
-    if (pc.bias != nullptr && pc.bias_row) rest.bias = (const char*)pc.bias + pc.m_main * esz;
-    const int st = run(head, workspace, workspace_bytes, s);
-    return st != CMPEXT3_OK ? st : run(rest, workspace, workspace_bytes, s);
-  }
-  if (plan.ws_bytes > 0 && (workspace == nullptr || align_of(workspace) < 16 || workspace_bytes < plan.ws_bytes))
-    return CMPEXT3_ERR_WORKSPACE;
-  const int dtype = pc.r.dtype, b_layout = pc.r.layout;
-  const int M = (int)pc.r.M, N = (int)pc.r.N, batch = (int)pc.r.batch;
-  int K = (int)pc.r.K;
-  const void* A = pc.A;
-  const void* B = pc.B;
-  int64_t lda = pc.r.lda, ldb = pc.r.ldb, stride_a = pc.r.stride_a, stride_b = pc.r.stride_b;
-  const int64_t esz = dtype == kF32 ? 4 : 2;
-  char* ws = (char*)workspace;
-  const bool kn = b_layout == CMPEXT3_B_KN;
-  if (plan.pad_a) {
-    const int64_t copies = (batch > 1 && stride_a != 0) ? batch : 1;
-    const hipError_t e = launch_pad_copy(A, lda, stride_a, M, K, ws, plan.lda_p, plan.stride_a_p, M, (int)plan.kp,
-                                         copies, (int)esz, s);
-    if (e != hipSuccess) return (int)e;
-    A = ws;
-    lda = plan.lda_p;
-    stride_a = plan.stride_a_p;
-    ws += plan.pad_a_bytes;
-  }
-  if (plan.pad_b) {
-    const int64_t copies = (batch > 1 && stride_b != 0) ? batch : 1;
-    const int rows = kn ? K : N, cols = kn ? N : K;
-    const int dst_rows = kn ? (int)plan.kp : N;
-    const hipError_t e = launch_pad_copy(B, ldb, stride_b, rows, cols, ws, plan.ldb_p, plan.stride_b_p, dst_rows,
-                                         (int)plan.ldb_p, copies, (int)esz, s);
-    if (e != hipSuccess) return (int)e;
-    B = ws;
-    ldb = plan.ldb_p;
-    stride_b = plan.stride_b_p;
-    ws += plan.pad_b_bytes;
-  }
-  if (plan.pad_a || plan.pad_b) K = (int)plan.kp;
+// Two launches share the workspace, one after the other (after the padded copies).
+int64_t workspace_need(const Prepared& pc) {
+  return pc.m_main > 0 || pc.n_main > 0 ? std::max(pc.plan.ws_bytes, pc.tail.ws_bytes) : pc.plan.ws_bytes;
+}
+
+// The operands that the kernels read (padded copies where the plan makes them) and the
+// part of C that they write.
+struct Operands {
+  const char* A;
+  const char* B;
+  char* C;
+  const char* bias;
+  int64_t lda, ldb, stride_a, stride_b;
+  int64_t M, N, K;
+};
+
+// Launches one plan's kernel(s), batch entries in chunks of at most 65535 grid rows.
+int launch_part(const Prepared& pc, const Plan& plan, const Operands& o, char* ws, hipStream_t s) {
+  const int64_t esz = pc.r.dtype == kF32 ? 4 : 2;
   GemmParams p{};
-  p.bias = pc.bias;
+  p.bias = o.bias;
   p.bias_row = pc.bias_row;
   p.b_dword = plan.b_dword;
-  p.bias_vec = pc.bias != nullptr && align_of(pc.bias) >= 8;
-  p.lda = lda;
-  p.ldb = ldb;
+  p.bias_vec = o.bias != nullptr && align_of(o.bias) >= 8;
+  p.lda = o.lda;
+  p.ldb = o.ldb;
   p.ldc = pc.r.ldc;
-  p.stride_a = stride_a;
-  p.stride_b = stride_b;
+  p.stride_a = o.stride_a;
+  p.stride_b = o.stride_b;
   p.stride_c = pc.r.stride_c;
-  p.M = M;
-  p.N = N;
-  p.K = K;
+  p.M = (int)o.M;
+  p.N = (int)o.N;
+  p.K = (int)o.K;
   p.tiles_m = plan.tiles_m;
   p.tiles_n = plan.tiles_n;
   p.group_m = plan.group_m;
@@ -274,16 +245,73 @@ int run(const Prepared& pc, void* workspace, int64_t workspace_bytes, hipStream_
                      plan.kernel == kF32Tile64K4 || plan.kernel == kF32Tile16K4 || plan.kernel == kSkinnyNK ||
                      plan.kernel == kTall;
   const int64_t zmax = kMaxGridZ / std::max(1, split_z ? plan.splits : 1);
-  for (int64_t b0 = 0; b0 < batch; b0 += zmax) {
-    const int64_t nb = std::min<int64_t>(zmax, batch - b0);
-    p.A = (const char*)A + b0 * stride_a * esz;
-    p.B = (const char*)B + b0 * stride_b * esz;
-    p.C = (char*)pc.C + b0 * pc.r.stride_c * esz;
+  for (int64_t b0 = 0; b0 < pc.r.batch; b0 += zmax) {
+    const int64_t nb = std::min<int64_t>(zmax, pc.r.batch - b0);
+    p.A = o.A + b0 * o.stride_a * esz;
+    p.B = o.B + b0 * o.stride_b * esz;
+    p.C = o.C + b0 * pc.r.stride_c * esz;
     const dim3 grid((unsigned)(plan.tiles_m * plan.tiles_n), 1, (unsigned)nb);
-    const hipError_t e = dispatch(plan, dtype, b_layout, p, grid, ws, s);
+    const hipError_t e = dispatch(plan, pc.r.dtype, pc.r.layout, p, grid, ws, s);
     if (e != hipSuccess) return (int)e;
   }
   return CMPEXT3_OK;
+}
+
+// Enqueues a prepared call: the zero-padded operand copies it planned, then its kernel(s).
+int run(const Prepared& pc, void* workspace, int64_t workspace_bytes, hipStream_t s) {
+  const Plan& plan = pc.plan;
+  if (pc.empty) return CMPEXT3_OK;
+  const int64_t need = workspace_need(pc);
+  if (need > 0 && (workspace == nullptr || align_of(workspace) < 16 || workspace_bytes < need))
+    return CMPEXT3_ERR_WORKSPACE;
+  const int M = (int)pc.r.M, N = (int)pc.r.N, K = (int)pc.r.K;
+  const int64_t batch = pc.r.batch;
+  const int64_t esz = pc.r.dtype == kF32 ? 4 : 2;
+  const bool kn = pc.r.layout == CMPEXT3_B_KN;
+  Operands o{(const char*)pc.A, (const char*)pc.B, (char*)pc.C, (const char*)pc.bias, pc.r.lda, pc.r.ldb,
+             pc.r.stride_a, pc.r.stride_b, M, N, K};
+  char* ws = (char*)workspace;
+  if (plan.pad_a) {
+    const int64_t copies = (batch > 1 && o.stride_a != 0) ? batch : 1;
+    const hipError_t e = launch_pad_copy(o.A, o.lda, o.stride_a, M, K, ws, plan.lda_p, plan.stride_a_p, M,
+                                         (int)plan.kp, copies, (int)esz, s);
+    if (e != hipSuccess) return (int)e;
+    o.A = ws;
+    o.lda = plan.lda_p;
+    o.stride_a = plan.stride_a_p;
+    ws += plan.pad_a_bytes;
+  }
+  if (plan.pad_b) {
+    const int64_t copies = (batch > 1 && o.stride_b != 0) ? batch : 1;
+    const int rows = kn ? K : N, cols = kn ? N : K;
+    const int dst_rows = kn ? (int)plan.kp : N;
+    const hipError_t e = launch_pad_copy(o.B, o.ldb, o.stride_b, rows, cols, ws, plan.ldb_p, plan.stride_b_p, dst_rows,
+                                         (int)plan.ldb_p, copies, (int)esz, s);
+    if (e != hipSuccess) return (int)e;
+    o.B = ws;
+    o.ldb = plan.ldb_p;
+    o.stride_b = plan.stride_b_p;
+    ws += plan.pad_b_bytes;
+  }
+  if (plan.pad_a || plan.pad_b) o.K = plan.kp;
+  if (pc.m_main <= 0 && pc.n_main <= 0) return launch_part(pc, plan, o, ws, s);
+  // two launches, one after the other on the stream
+  Operands head = o, rest = o;
+  if (pc.m_main > 0) {
+    head.M = pc.m_main;
+    rest.M -= pc.m_main;
+    rest.A += pc.m_main * o.lda * esz;
+    rest.C += pc.m_main * pc.r.ldc * esz;
+    if (o.bias != nullptr && pc.bias_row) rest.bias += pc.m_main * esz;
+  } else {
+    head.N = pc.n_main;
+    rest.N -= pc.n_main;
+    rest.B += pc.n_main * (kn ? 1 : o.ldb) * esz;
+    rest.C += pc.n_main * esz;
+    if (o.bias != nullptr && !pc.bias_row) rest.bias += pc.n_main * esz;
+  }
+  const int st = launch_part(pc, plan, head, ws, s);
+  return st != CMPEXT3_OK ? st : launch_part(pc, pc.tail, rest, ws, s);
 }
 
 // Shared body of cmpext3_gemm_ex (bias per column) and cmpext3_conv2d_1x1
@@ -326,15 +354,14 @@ extern "C" int cmpext3_gemm_prepare(cmpext3_gemm_call* call, int dtype, int b_la
 extern "C" int64_t cmpext3_gemm_call_workspace_size(const cmpext3_gemm_call* call) {
   const Prepared* pc = as_prepared(call);
   if (pc == nullptr) return (int64_t)CMPEXT3_ERR_INVALID_ARG;
-  // the two launches of a row split share the workspace, one after the other
-  return pc->m_main > 0 ? std::max(pc->plan.ws_bytes, pc->tail.ws_bytes) : pc->plan.ws_bytes;
+  return workspace_need(*pc);
 }
 
 extern "C" int cmpext3_gemm_call_describe(const cmpext3_gemm_call* call, char* buf, int buflen) {
   const Prepared* pc = as_prepared(call);
   if (pc == nullptr) return CMPEXT3_ERR_INVALID_ARG;
   if (buf && buflen > 0) {
-    const std::string d = describe_rows(pc->r, pc->plan, pc->m_main, pc->tail);
+    const std::string d = describe_parts(pc->r, pc->plan, pc->m_main, pc->n_main, pc->tail);
     strncpy(buf, d.c_str(), (size_t)buflen - 1);
     buf[buflen - 1] = '\0';
   }
@@ -422,8 +449,8 @@ extern "C" int64_t cmpext3_gemm_workspace_size(int dtype, int b_layout, int M, i
   Plan plan;
   const int st = make_plan(r, &plan);
   if (st != CMPEXT3_OK) return st;
-  RowSplit rs;
-  return plan_row_split(r, plan, &rs) ? std::max(rs.main.ws_bytes, rs.tail.ws_bytes) : plan.ws_bytes;
+  TwoPart two;
+  return plan_two_parts(r, plan, &two) ? std::max(two.main.ws_bytes, two.tail.ws_bytes) : plan.ws_bytes;
 }
 
 extern "C" int cmpext3_gemm_plan(int dtype, int b_layout, int M, int N, int K, int64_t lda, int64_t ldb,
@@ -433,14 +460,14 @@ extern "C" int cmpext3_gemm_plan(int dtype, int b_layout, int M, int N, int K, i
   Plan plan;
   const int st = make_plan(r, &plan);
   if (st != CMPEXT3_OK) return st;
-  RowSplit rs;
-  const bool split = M > 0 && N > 0 && batch > 0 && plan_row_split(r, plan, &rs);
+  TwoPart two;
+  const bool split = plan_two_parts(r, plan, &two);
   if (buf && buflen > 0) {
-    const std::string d = split ? describe_rows(r, rs.main, rs.m_main, rs.tail) : describe(r, plan);
+    const std::string d = split ? describe_parts(r, two.main, two.m_main, two.n_main, two.tail) : describe(r, plan);
     strncpy(buf, d.c_str(), (size_t)buflen - 1);
     buf[buflen - 1] = '\0';
   }
-  return (int)(split ? rs.main.kernel : plan.kernel);
+  return (int)(split ? two.main.kernel : plan.kernel);
 }
 
 extern "C" const char* cmpext3_status_string(int status) {

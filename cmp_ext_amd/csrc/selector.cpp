@@ -416,7 +416,7 @@ int make_plan_core(const Request& r, Plan* plan) {
     // column chunks
     const bool tall_ok = (r.align_a ? r.align_a : r.align) >= 16 && (r.align_b ? r.align_b : r.align) >= 16 &&
                          r.K % 8 == 0 && r.lda % 8 == 0 && r.ldb % 8 == 0 && r.N <= 128 &&
-                         (r.layout == kNK || r.N % 8 == 0) &&
+                         (r.layout == kNK || r.N % 8 == 0 || r.b_cols_padded) &&
                          (!batched || (r.stride_a % 8 == 0 && r.stride_b % 8 == 0));
     if (skinny_ok && !skinny_tiles_enough && r.layout == kNK) {
       // B is [N, K] (a Linear weight): strips of W rows.  With at most half as many strips
@@ -487,7 +487,7 @@ int make_plan_core(const Request& r, Plan* plan) {
       p.threads = r.M <= 64 ? 256 : 512;
     } else if (tall_ok && r.N <= 64 && r.M >= 1024 && r.K >= 1024 && cdiv(r.M, 128) * r.batch < kNumCUs &&
                (r.K <= 2048 ||
-                (r.K <= 4096 && (r.M * r.batch >= 8192 || (r.layout == kNK && r.N <= 32))))) {
+                (r.K <= 4096 && (r.M * r.batch >= 8192 || (r.layout == kNK && r.N <= 32) || r.N % 4 != 0)))) {
       // A narrow B (<= 64 columns) under fewer 128-row tiles than CUs: the tile kernels would
       // split K (or leave CUs idle) to fill the GPU; strips of A's rows over all of K stream
       // A once instead (MI355X, fp16, best strip vs the selector's tile128x128 (+ split):
@@ -495,7 +495,8 @@ int make_plan_core(const Request& r, Plan* plan) {
       // 16.6 vs 25.0, 16384 x 16 x 4096 27.7 vs 30.7, attention's P V over 8 x 2048 x 2048
       // with 64 columns 18.8 vs 25.7; measured slower from K = 8192, with 64 < N <= 128, or
       // at K = 4096 below 8192 rows -- except B as [N, K] with <= 32 rows, on one or two
-      // 16-row blocks: 4096 x 16 x 4096 7.9 vs 10.8 us, 1024 x 32 x 4096 8.7 vs 9.4).  64-row strips once they give every CU one and K >=
+      // 16-row blocks: 4096 x 16 x 4096 7.9 vs 10.8 us, 1024 x 32 x 4096 8.7 vs 9.4 -- or N %
+      // 4 != 0, where a tile cannot split K: 3000 x 33 x 4000 24 vs 51).  64-row strips once they give every CU one and K >=
       // 2048, else 32-row strips.
       p = tall_plan(r, cdiv(r.M, 64) * r.batch >= kNumCUs && r.K >= 2048 ? 64 : 32, p.group_m);
     } else if (tall_ok && r.N <= 64 && r.M >= 1024 && r.K >= 8192 && cdiv(r.M, 32) * r.batch <= 64 &&
@@ -705,7 +706,7 @@ int make_plan(const Request& r, Plan* plan) {
 }
 
 
-// Modelled time (us) of a 16-bit plan, for comparing a row split with the plan it would
+// Modelled time (us) of a 16-bit plan, for comparing two launches with the plan they would
 // replace: the tile cost model above for the tiled kernels, and reading A and B and
 // writing C once at ~5 TB/s for the HBM-bound ones; ~2 us per launch.
 static double plan_us(const Request& r, const Plan& p) {
@@ -717,8 +718,8 @@ static double plan_us(const Request& r, const Plan& p) {
   return bytes / 5.0e6 + 3.0;
 }
 
-bool plan_row_split(const Request& r, const Plan& full, RowSplit* out) {
-  if ((r.dtype != kF16 && r.dtype != kBF16) || full.forced || full.pad_a || full.pad_b || r.M <= 256 ||
+bool plan_two_parts(const Request& r, const Plan& full, TwoPart* out) {
+  if ((r.dtype != kF16 && r.dtype != kBF16) || full.forced || (r.M <= 256 && r.N <= 256) || r.M == 0 ||
       r.N == 0 || r.K == 0 || r.batch == 0)
     return false;
   const Candidate* fc = nullptr;
@@ -734,32 +735,82 @@ bool plan_row_split(const Request& r, const Plan& full, RowSplit* out) {
   const int64_t wgs = (int64_t)full.tiles_m * full.tiles_n * r.batch * std::max(1, full.splits);
   const int64_t rem = wgs % slots;
   if (wgs <= slots || rem == 0 || 2 * rem > slots) return false;
-  // rows covered by whole rounds of the 256-row tiles (one workgroup per CU), and whole 256-row tiles
-  int64_t cand[3] = {r.M / 256 * 256, 0, 0};
+  // what both launches read: the operands, or the padded copies of them
+  Request q = r;
+  const int64_t pad_bytes = full.pad_a_bytes + full.pad_b_bytes;
+  if (full.pad_a) {
+    q.lda = full.lda_p;
+    q.stride_a = full.stride_a_p;
+    q.align_a = 16;
+  }
+  if (full.pad_b) {
+    q.ldb = full.ldb_p;
+    q.stride_b = full.stride_b_p;
+    q.align_b = 16;
+    q.b_cols_padded = r.layout == kKN;
+  }
+  if (full.pad_a || full.pad_b) {
+    q.K = full.kp;
+    q.ws_bytes = r.ws_bytes - pad_bytes;
+  }
+  q.b_dword = full.b_dword;
+  if (full.pad_a || full.pad_b || full.b_dword) q.align = 16;  // (of A, of C, and of B where it counts)
+  // Cutting columns, and cutting padded operands, as rows of aligned ones: MI355X, one
+  // launch -> two, bf16 4095 x 4097 x 4096 203 -> 143 us (one column left), 8014 x 2506 x
+  // 1560 117.6 -> 68.0, 2702 x 7207 x 4533 280 -> 204, linear 2813 x 6272 x 3584 133.9 ->
+  // 114.3; of 22 random shapes 20 gained 2 to 42 % and two lost 1 and 3 %.
+  // Rows covered by whole rounds of the 256-row tiles (one workgroup per CU), and whole
+  // 256-row tiles; columns covered by whole rounds of 256- and 224-column tiles
+  struct Cut {
+    int64_t m, n;
+  } cuts[5] = {{r.M / 256 * 256, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}};
   for (int i = 0; i < 2; ++i) {
-    const int64_t cols = cdiv(r.N, i == 0 ? 256 : 224) * r.batch;
-    if (cols <= kNumCUs) {
-      const int64_t rows = 256 * (kNumCUs / cols);
-      cand[1 + i] = r.M / rows * rows;
+    const int64_t width = i == 0 ? 256 : 224;
+    const int64_t across = cdiv(r.N, width) * r.batch, down = cdiv(r.M, 256) * r.batch;
+    if (r.M > 256 && across <= kNumCUs) {
+      const int64_t rows = 256 * (kNumCUs / across);
+      cuts[1 + i].m = r.M / rows * rows;
+    }
+    if (r.N > 256 && down <= kNumCUs) {
+      const int64_t cols = width * (kNumCUs / down);
+      cuts[3 + i].n = r.N / cols * cols;
     }
   }
-  const double full_us = plan_us(r, full);
+  const double full_us = plan_us(q, full);
   double best = 0.92 * full_us;
   bool found = false;
-  for (int64_t m_main : cand) {
-    if (m_main <= 0 || m_main >= r.M) continue;
-    Request a = r, b = r;
-    a.M = m_main;
-    b.M = r.M - m_main;
-    // (the tail's A and C start m_main rows in: 16-byte aligned as the rows are, m_main
-    // being a multiple of 256)
+  for (const Cut& cut : cuts) {
+    if (cut.m >= r.M || cut.n >= r.N || cut.m + cut.n <= 0) continue;
+    Request a = q, b = q;
+    if (cut.m > 0) {
+      a.M = cut.m;
+      b.M = r.M - cut.m;
+    } else {
+      a.N = cut.n;
+      b.N = r.N - cut.n;
+    }
+    // (the tail's A and C start m rows in, or its B and C n columns in, multiples of 32: as
+    // aligned as the whole operands)
     Plan pa, pb;
-    if (make_plan(a, &pa) != CMPEXT3_OK || make_plan(b, &pb) != CMPEXT3_OK) continue;
-    if (pa.pad_a || pa.pad_b || pb.pad_a || pb.pad_b || pa.kernel == kGeneric16 || pb.kernel == kGeneric16) continue;
+    if (make_plan_core(a, &pa) != CMPEXT3_OK || make_plan_core(b, &pb) != CMPEXT3_OK) continue;
+    if (pa.kernel == kGeneric16 || pb.kernel == kGeneric16) continue;
     const double us = plan_us(a, pa) + plan_us(b, pb);
     if (us < best) {
       best = us;
-      out->m_main = m_main;
+      out->m_main = cut.m;
+      out->n_main = cut.n;
+      pa.b_dword = pb.b_dword = full.b_dword;
+      pa.pad_a = full.pad_a;
+      pa.pad_b = full.pad_b;
+      pa.kp = full.kp;
+      pa.lda_p = full.lda_p;
+      pa.ldb_p = full.ldb_p;
+      pa.stride_a_p = full.stride_a_p;
+      pa.stride_b_p = full.stride_b_p;
+      pa.pad_a_bytes = full.pad_a_bytes;
+      pa.pad_b_bytes = full.pad_b_bytes;
+      pa.ws_bytes += pad_bytes;
+      pb.ws_bytes += pad_bytes;
       out->main = pa;
       out->tail = pb;
       found = true;

@@ -51,17 +51,19 @@ struct Request {
 // Returns 0 and fills *plan, or a negative CMPEXT3_ERR_* code.
 int make_plan(const Request& r, Plan* plan);
 
-// A 16-bit tiled product whose last round of tiles would run mostly empty (rows just
-// past a multiple of what one round covers) runs as two launches over its rows: rows
-// [0, m_main) with `main`, the remaining rows with `tail` (each planned for its rows of
-// the same operands; they write disjoint rows of C).
-struct RowSplit {
-  int64_t m_main;
+// A 16-bit tiled product whose last round of tiles would run mostly empty (rows or columns
+// just past a multiple of what one round covers) runs as two launches, over rows
+// [0, m_main) with `main` and the remaining rows with `tail`, or over columns
+// [0, n_main) and the remaining ones (the other of the two is 0).  Each is planned for its
+// part of the same operands -- the padded copies, where `full` makes them, which `main`
+// then names and the workspace of both includes; they write disjoint parts of C.
+struct TwoPart {
+  int64_t m_main, n_main;
   Plan main, tail;
 };
-// Given the plan for all rows, returns true and fills *out when the two launches are
-// modelled to take less than 0.92 of its time.
-bool plan_row_split(const Request& r, const Plan& full, RowSplit* out);
+// Given the plan for the whole product, returns true and fills *out when the two launches
+// are modelled to take less than 0.92 of its time.
+bool plan_two_parts(const Request& r, const Plan& full, TwoPart* out);
 
 // One-line description of a plan, e.g. "tile256x256 f16 KN grid=256x1".
 std::string describe(const Request& r, const Plan& p);

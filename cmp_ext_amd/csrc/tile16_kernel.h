@@ -318,6 +318,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const G
     });
     return;
   }
+  typedef u32x4 u32x4_e2 __attribute__((aligned(2)));
   T* Cb = (T*)p.C + bz * p.stride_c;
   const uint16_t* bias = (const uint16_t*)p.bias;
   // store width C's rows allow (every batch entry's): 16 bytes, 8 bytes, or one element
@@ -392,6 +393,8 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const G
           } else if (n + 8 <= N && st8) {  // 8-byte aligned rows
             *(u32x2*)dst = u32x2{v.x, v.y};
             *(u32x2*)(dst + 4) = u32x2{v.z, v.w};
+          } else if (n + 8 <= N) {  // rows of any pitch: one store all the same, aligned to an element
+            *(u32x4_e2*)dst = v;
           } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
