@@ -2,8 +2,8 @@
 //
 // Counterpart of gemm_fp32_ga100_kernel (src/cuda/fp32_matmul.cu:31-184):
 // same contract (row-major, any M/N/K, fully bounds-checked loads and stores),
-// but the products run on v_mfma_f32_16x16x4_f32 (fused multiply-add with fp32
-// accumulation) instead of the reference's separate __fmul_rn/__fadd_rn SIMT
+// but the products run on the matrix cores with fp32 accumulation (on the bf16
+// instruction, each float as three bf16 planes, or on v_mfma_f32_16x16x4_f32) instead of the reference's separate __fmul_rn/__fadd_rn SIMT
 // loop, which exists only to dodge a GA100 FMA limit (fp32_matmul.cu:20-26).
 //
 // Any alignment is accepted: global memory is read by 4-byte LDS-DMA
@@ -13,11 +13,9 @@
 // Operands whose rows are 16-byte aligned with K (and N for B given as [K,N])
 // a multiple of 4 use 16-byte LDS-DMA instead (DMA16: buffer_load_dwordx4 ...
 // lds, 1 KiB per instruction): a quarter of the load instructions and their
-// address work, measured 132 -> 142 TFLOP/s at 4096^3 on 128 x 128 tiles.  The
-// DMA fills a ring of NS stages of BK = 16 k; each wave counts its own DMA in
-// vmcnt, and one "s_waitcnt vmcnt; s_barrier" per step certifies that the
-// next stage is complete and that the slot about to be refilled is free, so
-// NS-2 stages of loads are always in flight without staging registers.
+// address work.  The DMA fills a ring of four stages of BK = 16 k, two at a time
+// while the two before are multiplied; one wait and barrier per pair certifies that the
+// next pair has landed and that every wave is done with the slots about to be refilled.
 //
 // LDS layouts (per stage):
 //   A, and B given as [N,K]: rows of 16 floats (64 bytes) in groups of 16 rows
@@ -31,18 +29,18 @@
 //     stored at segment s ^ ((k/4)%4): the fragment read of MFMA step s
 //     (rows s, 4+s, 8+s, 12+s at 16 columns, ds_read_b32) hits 64 distinct
 //     banks, and one DMA instruction writes 64 consecutive floats of a row.
-// MFMA k-step s of lane group g uses k = 4g + s, so one ds_read_b128 per A
-// fragment feeds four MFMAs.
+// Lane group g holds k = 4g .. 4g+3 of a stage (one ds_read_b128 of A): the eight k of a
+// bf16 instruction's lane come from a pair of stages, four fp32 instructions use one each.
 #pragma once
 
 #include "device_common.h"
 
 namespace cmpext3 {
 
-template <int BM, int BN, int NS_, bool DMA16 = false>
+template <int BM, int BN, bool DMA16 = false>
 struct F32Shape {
   static constexpr int BK = 16;
-  static constexpr int NS = NS_;
+  static constexpr int NS = 4;    // ring slots, two stages loaded and two multiplied at a time
   static constexpr int NT = 256;  // 2 x 2 waves
   static constexpr int WTM = BM / 2, WTN = BN / 2;
   static constexpr int FM = WTM / 16, FN = WTN / 16;
@@ -54,10 +52,7 @@ struct F32Shape {
   // DMA16: 1 KiB instructions t = 4i + wave, i < A16 (B16), skipping t >= A_BYTES / 1024
   static constexpr int A16 = (A_BYTES / 1024 + 3) / 4;
   static constexpr int B16 = (B_BYTES / 1024 + 3) / 4;
-  static constexpr int DMA = DMA16 ? A16 + B16 : A_DMA + B_DMA;
   static_assert(BN % 64 == 0 && BM % 32 == 0, "whole DMA instructions per wave, 64-float B rows");
-  static_assert(!DMA16 || NS == 2, "DMA16 waves may issue different counts: vmcnt(0) only");
-  static_assert(NS >= 2 && (NS - 2) * DMA <= 63, "ring depth / vmcnt range");
   static_assert(NS * STAGE <= 160 * 1024, "LDS");
 };
 
@@ -84,17 +79,55 @@ __device__ __forceinline__ uint32_t f32_off(int row, int chunk) {
   return (uint32_t)((row >> 4) * 1024 + 16 * f32_slot(row & 15, chunk));
 }
 
-// WAVES: waves per SIMD the kernel is compiled for (caps its registers at 512 / WAVES).
-// Enough resident workgroups matter more than registers here: 96 x 64 tiles at 8
-// waves per SIMD run all 2021 tiles of a 4097 x 3001 product in one round (measured
-// 460 -> 421 us on MI355X against the compiler's choice of 7).
+// ---- fp32 products on the bf16 matrix cores ----
+// A float is the exact sum of three bf16 values: its top 16 bits (h), the top 16 bits of
+// what is left (m) and the rest (l), 8 significant bits each.  Of the nine products of
+// two such sums, six (h h, h m, m h, m m, h l, l h) are summed in fp32 by v_mfma_f32_
+// 16x16x32_bf16; the three left out are below 2^-23 of the product.  Sums of K products
+// take 6 roundings per 32 k where the fp32 instruction takes 8 (16x16x4), and the results
+// are closer to the exact ones (relative Frobenius error against float64: 4097 x 3001 x
+// 2049 uniform 8.1e-7 -> 7.0e-7, 2048^3 normal 5.7e-7 -> 4.9e-7, 1024^2 x 8192 positive
+// 1.6e-7 -> 1.5e-7).  What the planes cannot hold -- infinities (their m is a NaN) and
+// values with bits below bf16's smallest (under 2^-110 or so) -- is seen in the sums or in
+// l's dropped bits, and the tile is then computed again on the fp32 instruction.
+// Splitting an element takes ~6 vector instructions in each wave that reads it, as many
+// cycles as its products where a wave's block is small: that bounds the 96 x 64 and 64 x
+// 64 tiles (rounding instead of cutting off took longer, 12 cycles a conversion; one wave
+// per K stage, which splits less, left too few waves).  MI355X, fp32 instruction -> this:
+// 4096^3 (128 x 128) 949 -> 692 us, 4097 x 3001 x 2049 (96 x 64, 4-byte DMA) 396 -> 357,
+// 4100 x 3000 x 2048 (96 x 64) 371 -> 325, 3000 x 2000 x 1000 (64 x 64) 101 -> 96.
+struct F32Planes {
+  u32x4 h, m, l;  // 8 k: two 16-k stages of 4
+};
+// The planes of eight floats; bits that bf16 drops from l go to `lost`.
+__device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y, uint32_t& lost) {
+  F32Planes p;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 v = i < 2 ? x : y;
+    const float a = v[2 * (i & 1)], b = v[2 * (i & 1) + 1];
+    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+    const float ra = a - __uint_as_float(ua & 0xFFFF0000u), rb = b - __uint_as_float(ub & 0xFFFF0000u);
+    const uint32_t va = __float_as_uint(ra), vb = __float_as_uint(rb);
+    const uint32_t wa = __float_as_uint(ra - __uint_as_float(va & 0xFFFF0000u));
+    const uint32_t wb = __float_as_uint(rb - __uint_as_float(vb & 0xFFFF0000u));
+    p.h[i] = pack_hi16(ua, ub);
+    p.m[i] = pack_hi16(va, vb);
+    p.l[i] = pack_hi16(wa, wb);
+    // (in asm: as C++ the ORs were put off to the end, with every w kept in a register)
+    asm volatile("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(wa), "v"(wb));
+  }
+  return p;
+}
+
 // SPLITK: grid.z = batch * p.splits; this workgroup sums its split's K range and
 // stores the sums into p.partials (bias added by the reduction).
-template <bool KN, int BM, int BN, int NS, int WAVES, bool SPLITK = false, bool DMA16 = false>
-__global__ void __launch_bounds__(256, WAVES) gemm_f32_kernel(const GemmParams p) {
-  using S = F32Shape<BM, BN, NS, DMA16>;
-  constexpr int FM = S::FM, FN = S::FN;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[NS * S::STAGE];
+// EXACT: on the fp32 instruction.  Otherwise returns true, with nothing written, when the
+// tile needs that (see above).
+template <bool KN, int BM, int BN, bool SPLITK, bool DMA16, bool EXACT>
+__device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* smem) {
+  using S = F32Shape<BM, BN, DMA16>;
+  constexpr int FM = S::FM, FN = S::FN, NS = S::NS;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -241,55 +274,110 @@ __global__ void __launch_bounds__(256, WAVES) gemm_f32_kernel(const GemmParams p
   const uint32_t fb_kn = S::A_BYTES + (uint32_t)(4 * g * BN * 4 + 4 * r16);
 
   f32x4 acc[FM][FN];
+  // This wave's fragments of a stage (4 k per lane: k = 4g .. 4g+3)
+  auto read_a = [&](int slot, int i) { return *(const f32x4*)(smem + slot * S::STAGE + fa + i * 1024); };
+  auto read_b = [&](int slot, int j) {
+    const unsigned char* stage = smem + slot * S::STAGE;
+    if (!KN) return *(const f32x4*)(stage + fb_nk + j * 1024);
+    f32x4 x;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = *(const float*)(stage + fb_kn + s * BN * 4 + (((wn * FN + j) ^ g) << 6));
+    return x;
+  };
+
+  // Stages in ring slots slot and slot + 1 (32 k) on the bf16 instruction: B's next block is
+  // split while the current one's products run, the small products first.
+  uint32_t lost = 0;
+  auto split_pair = [&](int slot) {
+    F32Planes pa[FM], pb[FN];
+    f32x4 y0[FN], y1[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      y0[j] = read_b(slot, j);
+      y1[j] = read_b(slot + 1, j);
+    }
+#pragma unroll
+    for (int i = 0; i < FM; ++i) pa[i] = f32_split(read_a(slot, i), read_a(slot + 1, i), lost);
+    pb[0] = f32_split(y0[0], y1[0], lost);
+    static_for<FN>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (j + 1 < FN) pb[j + 1] = f32_split(y0[j + 1], y1[j + 1], lost);
+      auto product = [&](u32x4 F32Planes::*b, u32x4 F32Planes::*a) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i) acc[i][j] = Mfma<__bf16>::mma(pb[j].*b, pa[i].*a, acc[i][j]);
+      };
+      product(&F32Planes::l, &F32Planes::h);
+      product(&F32Planes::h, &F32Planes::l);
+      product(&F32Planes::m, &F32Planes::m);
+      product(&F32Planes::m, &F32Planes::h);
+      product(&F32Planes::h, &F32Planes::m);
+      product(&F32Planes::h, &F32Planes::h);
+      if constexpr (j + 1 < FN) {
+        static_for<6 * FM>([&](auto) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one product,
+          __builtin_amdgcn_sched_group_barrier(0x002, (48 + 6 * FM - 1) / (6 * FM), 0);  // its share of the splitting
+        });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  auto exact_stage = [&](int slot) {  // on the fp32 instruction
+    f32x4 x[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) x[i] = read_a(slot, i);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const f32x4 y = read_b(slot, j);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < FM; ++i) acc[i][j] = mma_f32(y[s], x[i][s], acc[i][j]);
+    }
+  };
+  // every load has landed and every wave's reads are done
+  auto certify = [&]() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
+
+  // Two stages at a time: stages st+2 and st+3 (zeros past K) load into the slots that the
+  // iteration before read while st and st+1 are multiplied.
+  const int nst = (K + S::BK - 1) / S::BK;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto compute_stage = [&](int st) {
-    const unsigned char* stage = smem + (st % NS) * S::STAGE;
-    f32x4 af[FM];
-#pragma unroll
-    for (int i = 0; i < FM; ++i) af[i] = *(const f32x4*)(stage + fa + i * 1024);
-    if (KN) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        float bf[FN];
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          bf[j] = *(const float*)(stage + fb_kn + s * BN * 4 + (((wn * FN + j) ^ g) << 6));
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] = mma_f32(bf[j], af[i][s], acc[i][j]);
-      }
-    } else {
-      f32x4 bf[FN];
-#pragma unroll
-      for (int j = 0; j < FN; ++j) bf[j] = *(const f32x4*)(stage + fb_nk + j * 1024);
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] = mma_f32(bf[j][s], af[i][s], acc[i][j]);
-    }
-  };
-  auto certify = [&]() {
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NS - 2) * S::DMA) : "memory");
-  };
-
-  const int nst = (K + S::BK - 1) / S::BK;
-  // Step st: DMA stage st+NS-1 (zeros past K), compute st, certify st+1.
-#pragma unroll
-  for (int t = 0; t < NS - 1; ++t) load_stage(t);
+  load_stage(0);
+  load_stage(1);
   certify();
-  for (int st = 0; st < nst; ++st) {
-    load_stage(st + NS - 1);
-    compute_stage(st);
+  for (int st = 0; st < nst; st += 2) {
+    const int slot = st & 2;
+    load_stage(st + 2);
+    load_stage(st + 3);
+    if constexpr (EXACT) {
+      exact_stage(slot);
+      exact_stage(slot + 1);
+    } else {
+      split_pair(slot);
+    }
     certify();
   }
-  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // no LDS DMA may outlive the workgroup
+  if constexpr (!EXACT) {
+    bool again = (lost & 0xFFFFu) != 0;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) again |= !(__builtin_fabsf(acc[i][j][e]) <= 3.402823466e+38f);
+    // (through the ring, which is free: __syncthreads_or's own LDS would cost the 96 x 64 tile
+    // its fourth workgroup per CU)
+    uint32_t* any = (uint32_t*)smem;
+    const uint64_t lanes = __ballot(again);
+    if (lane == 0) any[wave] = lanes != 0;
+    __syncthreads();
+    const uint32_t redo = any[0] | any[1] | any[2] | any[3];
+    __syncthreads();
+    if (redo) return true;
+  }
 
   if constexpr (SPLITK) {  // fp32 partial sums, four consecutive columns per store (N % 4 == 0)
     const int batch = (int)gridDim.z / p.splits;
@@ -303,7 +391,7 @@ __global__ void __launch_bounds__(256, WAVES) gemm_f32_kernel(const GemmParams p
         if (m < M && n < N) *(f32x4*)(part + (int64_t)m * N + n) = acc[i][j];
       }
     }
-    return;
+    return false;
   }
   // acc[i][j][e] = C[m0 + wm*WTM + 16i + r16][n0 + wn*WTN + 16j + 4g + e]; elements
   // outside C get an out-of-range offset and are dropped by the store.
@@ -336,7 +424,7 @@ __global__ void __launch_bounds__(256, WAVES) gemm_f32_kernel(const GemmParams p
         buf_store16(crs, row_ok && n0 + col < N ? (uint32_t)(row * p.ldc + col) * 4u : kBufOOB, v);
       }
     }
-    return;
+    return false;
   }
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
@@ -355,6 +443,15 @@ __global__ void __launch_bounds__(256, WAVES) gemm_f32_kernel(const GemmParams p
       }
     }
   }
+  return false;
+}
+
+// WAVES: waves per SIMD the kernel is compiled for (caps its registers at 512 / WAVES).
+template <bool KN, int BM, int BN, int WAVES, bool SPLITK = false, bool DMA16 = false>
+__global__ void __launch_bounds__(256, WAVES) gemm_f32_kernel(const GemmParams p) {
+  using S = F32Shape<BM, BN, DMA16>;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[S::NS * S::STAGE];
+  if (f32_tile<KN, BM, BN, SPLITK, DMA16, false>(p, smem)) f32_tile<KN, BM, BN, SPLITK, DMA16, true>(p, smem);
 }
 
 }  // namespace cmpext3

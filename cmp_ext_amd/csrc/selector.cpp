@@ -58,18 +58,19 @@ const Candidate kTiles16[] = {
     {kTile256x224, 256, 224, 1, 0.98, 0.98},
     {kTile128x128, 128, 128, 2, 0.81, 0.57},
 };
-// fp32 tiles.  A CU holds up to `occ` of their workgroups at once and shares its
-// matrix cores among them; how busy it keeps them grows with the number it holds:
-// from u1 (one workgroup, latency-bound) to umax (occ of them).  Fitted on MI355X to
-// 345 timed (tile, K split) choices over 27 shapes (M 16..4097, N 1024..4096, K
-// 1024..14336): the model's choice is within 1.7 % of the fastest measured one
-// (geometric mean; worst 1.18x at 1024^3), against 1.12x for a model with a fixed
-// per-tile efficiency.  The 4-byte LDS-DMA path (rows not 16-byte aligned) scales
-// umax by dma4, measured per tile at full occupancy against the 16-byte path on the
-// same box: 128x128 505 vs 539 us, 96x64 412 vs 423, 64x64 270 vs 321.  64x64k4 (K
-// split over the four waves, two workgroups per CU) fitted the same way to 114 more
-// timings: u1 0.62, umax 0.72; with it the model's choice is within 0.4 % of the
-// fastest measured (tile, split) over those 29 shapes.  16x64k4 (M <= 16, bound by
+// fp32 tiles.  A CU holds several of their workgroups at once and shares its matrix
+// cores among them; how busy it keeps them grows with the number it holds: from u1 (one
+// workgroup, latency-bound) to umax (occ of them and more), in units of the fp32
+// instruction's rate, which 128x128, 96x64 and 64x64 can exceed (they run on the bf16
+// instruction, f32_kernel.h).  Their numbers follow timings of every tile with 1, 2, 3,
+// 4 and 8 K splits on 15 shapes (MI355X; M 64..4097, N 1000..4096, K 500..8192): 128x128,
+// whose waves split the fewest operand elements per product, 1.0 alone and 1.09..1.25 in
+// pairs, 96x64 0.65 alone and 0.93..0.98 with four to eight, 64x64 0.45..0.55 and
+// 0.84..0.89.  Its choices against the ones before, on the same kernels: 512 x 4096 x 4096
+// 139.5 -> 106.7 us (128x128 in 4 splits for 64x64 in 4), 2048^3 136 -> 104, 384 columns
+// x[1997, 3840] 60 -> 47.7.  The 4-byte LDS-DMA path (rows not 16-byte aligned) scales
+// umax by dma4.  64x64k4 (K split over the four waves, two workgroups per CU; fp32
+// instruction) was fitted to 114 timings: u1 0.62, umax 0.72; 16x64k4 (M <= 16, bound by
 // streaming B) to 134 more over 29 shapes with M <= 16: u1 0.36, umax 0.46, and a CU
 // streams its workgroups' B strips at ~19 GB/s with one of them, ~24 GB/s with more
 // (6 TB/s over 256 CUs); the choice is then within 2.7 % of the fastest measured.
@@ -78,13 +79,14 @@ struct F32Tile {
   int bm, bn, occ;
   double u1, umax, dma4;
   int kwaves;  // waves that split a workgroup's 16-k steps among them
+  int lead;    // steps that filling its ring and storing its tile cost a CU's last one
 };
 const F32Tile kTiles32[] = {
-    {kF32Tile128, 128, 128, 4, 0.75, 0.94, 0.937, 1},
-    {kF32Tile96x64, 96, 64, 8, 0.50, 0.89, 0.975, 1},
-    {kF32Tile64, 64, 64, 8, 0.44, 0.875, 0.84, 1},
-    {kF32Tile64K4, 64, 64, 2, 0.62, 0.72, 0.84, 4},
-    {kF32Tile16K4, 16, 64, 4, 0.36, 0.46, 0.84, 4},
+    {kF32Tile128, 128, 128, 2, 0.95, 1.14, 0.82, 1, 2},
+    {kF32Tile96x64, 96, 64, 8, 0.655, 0.95, 0.975, 1, 1},
+    {kF32Tile64, 64, 64, 3, 0.45, 0.845, 0.84, 1, 1},
+    {kF32Tile64K4, 64, 64, 2, 0.62, 0.72, 0.84, 4, 0},
+    {kF32Tile16K4, 16, 64, 4, 0.36, 0.46, 0.84, 4, 4},
 };
 // Modelled microseconds: w = workgroups on the busiest CU, each running cdiv(K/s, 16)
 // steps of bm*bn*16 MFMA work (bm*bn*32 / (256 * 2380) us at the full fp32 rate of a
@@ -99,7 +101,7 @@ double f32_cost(const F32Tile& c, int64_t M, int64_t N, int64_t K, int64_t batch
   const double u = c.u1 + (umax - c.u1) * std::min(1.0, (double)(w - 1) / (c.occ - 1));
   const double mem = std::max((double)batch * (M * K + K * N) * 4.0 / 5.4e6,
                               (double)w * c.bn * cdiv(K, s) * 4.0 / (w == 1 ? 19e3 : 24e3));
-  double t = 1.0 + std::max((double)w * steps * step_us / u, mem);
+  double t = 1.0 + std::max(((double)w * steps + c.lead) * step_us / u, mem);
   if (s > 1) t += (double)s * batch * M * N * 8.0 / 5.5e6 + 3.8;
   return t;
 }
