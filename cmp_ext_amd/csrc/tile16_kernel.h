@@ -163,10 +163,13 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile16_kernel(const G
       r[2] = live ? (int)kBufRecords : 0;
       // B as [K,N] with 4-byte aligned rows: a row's last piece may run into the next row
       // (columns >= N, which are not stored), the last row's past the operand, so the
-      // descriptor ends where the operand does (the range check is per dword)
+      // descriptor ends with the dword that holds the operand's last element (a dword is
+      // loaded when all of it is in range, zeros otherwise; where N is odd that dword's other
+      // half is column N, not stored either)
       if constexpr (KN && check) {
         if (live && p.b_dword) {
-          const int64_t bytes = ((int64_t)(p.K - kbeg - k0 - 1) * ldb + (N - n0)) * (int64_t)sizeof(T);
+          const int64_t elems = (int64_t)(p.K - kbeg - k0 - 1) * ldb + (N - n0);
+          const int64_t bytes = (elems * (int64_t)sizeof(T) + 3) & ~(int64_t)3;
           r[2] = bytes < (int64_t)kBufRecords ? (int)bytes : (int)kBufRecords;
         }
       }

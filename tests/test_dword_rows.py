@@ -75,3 +75,37 @@ def test_results(dtype, M, N, K, gap, off, batch):
     assert "b_dword" in desc, desc
     for i in range(batch):
         assert O.reference_check(out[i].cpu(), a[i], b[i], dtype) <= O.TOLERANCE[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K,gap,off,batch", [
+    (512, 1001, 1024, 1, 0, 1), (200, 1003, 264, 3, 2, 1), (130, 999, 136, 5, 6, 2), (300, 129, 2048, 1, 0, 1),
+    (4095, 4097, 64, 1, 0, 1), (200, 1001, 1024, 7, 0, 1), (512, 1002, 1024, 0, 0, 1), (130, 1004, 136, 2, 2, 2),
+])
+def test_last_column_of_the_last_row(dtype, M, N, K, gap, off, batch):
+    """B's last element, at the very end of the operand (in the middle of a dword where N is
+    odd and the pitch even), outweighs the rest of its column, with NaN after it: the last
+    columns element by element."""
+    import cmpext3
+
+    dt = {"fp16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    g = torch.Generator().manual_seed(N + K)
+    a = torch.rand((batch, M, K), generator=g).add_(0.5).to(dt)
+    b = (torch.randn((batch, K, N), generator=g) / K).to(dt)
+    b[:, K - 1] *= 64
+    b[:, K - 1, N - 1] = 7
+    ldb = N + gap
+    buf = torch.full((off + batch * K * ldb,), float("nan"), dtype=dt, device="cuda")
+    view = buf[off:].view(batch, K, ldb)[:, :, :N]
+    view.copy_(b)
+    matmul = cmpext3.fp16_matmul if dtype == "fp16" else cmpext3.bf16_matmul
+    out = matmul(a[0].cuda(), view[0])[None] if batch == 1 else cmpext3.bmm(a.cuda(), view)
+    desc = cmpext3.last_plan()
+    print(dtype, M, N, K, gap, off, batch, desc, flush=True)
+    assert "b_dword" in desc, desc
+    a, b = a.double(), b[:, :, N - 9 :].double()
+    ref, size = a @ b, a @ b.abs()
+    # fp32 sums of K products and one rounding to 11 or 8 bits
+    bound = K * 2.0 ** -24 * size + 2.0 ** (-11 if dtype == "fp16" else -8) * ref.abs() + 2.0 ** -24
+    assert ((out[:, :, N - 9 :].double().cpu() - ref).abs() <= bound).all()
