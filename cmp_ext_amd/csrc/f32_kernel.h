@@ -3,8 +3,9 @@
 // Counterpart of gemm_fp32_ga100_kernel (src/cuda/fp32_matmul.cu:31-184):
 // same contract (row-major, any M/N/K, fully bounds-checked loads and stores),
 // but the products run on the matrix cores with fp32 accumulation (on the bf16
-// instruction, each float as three bf16 planes, or on v_mfma_f32_16x16x4_f32) instead of the reference's separate __fmul_rn/__fadd_rn SIMT
-// loop, which exists only to dodge a GA100 FMA limit (fp32_matmul.cu:20-26).
+// instruction, each float as three bf16 planes, or on v_mfma_f32_16x16x4_f32)
+// instead of the reference's separate __fmul_rn/__fadd_rn SIMT loop, which exists
+// only to dodge a GA100 FMA limit (fp32_matmul.cu:20-26).
 //
 // Any alignment is accepted: global memory is read by 4-byte LDS-DMA
 // (buffer_load_dword ... lds, 256 contiguous LDS bytes per instruction), with
@@ -37,7 +38,7 @@
 
 namespace cmpext3 {
 
-template <int BM, int BN, bool DMA16 = false>
+template <int BM, int BN>
 struct F32Shape {
   static constexpr int BK = 16;
   static constexpr int NS = 4;    // ring slots, two stages loaded and two multiplied at a time
@@ -80,22 +81,32 @@ __device__ __forceinline__ uint32_t f32_off(int row, int chunk) {
 }
 
 // ---- fp32 products on the bf16 matrix cores ----
-// A float is the exact sum of three bf16 values: its top 16 bits (h), the top 16 bits of
-// what is left (m) and the rest (l), 8 significant bits each.  Of the nine products of
-// two such sums, six (h h, h m, m h, m m, h l, l h) are summed in fp32 by v_mfma_f32_
-// 16x16x32_bf16; the three left out are below 2^-23 of the product.  Sums of K products
-// take 6 roundings per 32 k where the fp32 instruction takes 8 (16x16x4), and the results
-// are closer to the exact ones (relative Frobenius error against float64: 4097 x 3001 x
-// 2049 uniform 8.1e-7 -> 7.0e-7, 2048^3 normal 5.7e-7 -> 4.9e-7, 1024^2 x 8192 positive
-// 1.6e-7 -> 1.5e-7).  What the planes cannot hold -- infinities (their m is a NaN) and
+// A float x is the exact sum of three bf16 values: h, x rounded to 8 significant bits, m,
+// the top 8 bits of the signed rest, and l, what is left.  Of the nine products of two
+// such sums, six are summed in fp32 by v_mfma_f32_16x16x32_bf16: h h in one accumulator,
+// the five small ones (h m, m h, m m, h l, l h, in sum about 2^-7 of h h) in another, so
+// that they are rounded at their own size, and the two are added at the end.  (In one
+// accumulator the instruction cut the small products off below the sum's last bits,
+// always the same way: sums of 8192 positive products were off by 1.6e-5, the fp32
+// instruction's by 1.2e-6.)  m l, l m and l l are left out, together at most 2^-23 of the
+// product, and m's sign is independent of x's, so that they do not add up.  A chain
+// rounds once per 32 k where the fp32 instruction's (16x16x4) rounds 8 times.  Relative
+// Frobenius error against float64 on MI355X, fp32 instruction -> this: 512 x 512 x 8192
+// normal 1.62e-6 -> 0.57e-6, positive (uniform in [0, 1)) 1.19e-6 -> 0.42e-6, x 2048
+// 8.1e-7 -> 2.7e-7 and 6.0e-7 -> 2.2e-7, x 128 2.0e-7 -> 0.67e-7, x 32 1.0e-7 -> 0.41e-7,
+// x 16 7.4e-8 -> 3.6e-8, x 4 4.0e-8 -> 3.0e-8; x 1 2.5e-8 (one rounding) -> 3.0e-8, the
+// only one of these that is larger.
+// What the planes cannot hold -- infinities, floats of 2^112 and more (their m is a NaN) and
 // values with bits below bf16's smallest (under 2^-110 or so) -- is seen in the sums or in
 // l's dropped bits, and the tile is then computed again on the fp32 instruction.
-// Splitting an element takes ~6 vector instructions in each wave that reads it, as many
+// Splitting an element takes 7 vector instructions in each wave that reads it, as many
 // cycles as its products where a wave's block is small: that bounds the 96 x 64 and 64 x
-// 64 tiles (rounding instead of cutting off took longer, 12 cycles a conversion; one wave
-// per K stage, which splits less, left too few waves).  MI355X, fp32 instruction -> this:
-// 4096^3 (128 x 128) 949 -> 692 us, 4097 x 3001 x 2049 (96 x 64, 4-byte DMA) 396 -> 357,
-// 4100 x 3000 x 2048 (96 x 64) 371 -> 325, 3000 x 2000 x 1000 (64 x 64) 101 -> 96.
+// 64 tiles (rounding by bf16 conversions took longer, 12 cycles each; one wave per K
+// stage, which splits less, left too few waves; sums of 32 k in registers of their own,
+// added to the total on the vector units, took 5 % longer than the two accumulators).
+// MI355X, fp32 instruction -> this: 4096^3 (128 x 128) 946 -> 760 us, 4097 x 3001 x 2049
+// (96 x 64, 4-byte DMA) 394 -> 396, 4100 x 3000 x 2048 (96 x 64) 369 -> 351, 3000 x 2000 x
+// 1000 (64 x 64) 101 -> 103.
 struct F32Planes {
   u32x4 h, m, l;  // 8 k: two 16-k stages of 4
 };
@@ -105,17 +116,23 @@ __device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y, uint32_t& lost)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const f32x4 v = i < 2 ? x : y;
-    const float a = v[2 * (i & 1)], b = v[2 * (i & 1) + 1];
-    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
-    const float ra = a - __uint_as_float(ua & 0xFFFF0000u), rb = b - __uint_as_float(ub & 0xFFFF0000u);
-    const uint32_t va = __float_as_uint(ra), vb = __float_as_uint(rb);
-    const uint32_t wa = __float_as_uint(ra - __uint_as_float(va & 0xFFFF0000u));
-    const uint32_t wb = __float_as_uint(rb - __uint_as_float(vb & 0xFFFF0000u));
-    p.h[i] = pack_hi16(ua, ub);
-    p.m[i] = pack_hi16(va, vb);
-    p.l[i] = pack_hi16(wa, wb);
-    // (in asm: as C++ the ORs were put off to the end, with every w kept in a register)
-    asm volatile("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(wa), "v"(wb));
+    uint32_t h[2], m[2], l[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float a = v[2 * (i & 1) + e];
+      // t = 2^16 a + a to 24 bits, so t - 2^16 a is a to 8 bits, exactly, and so is the rest
+      const float t = a * 65537.f;
+      const float hi = __builtin_fmaf(a, -65536.f, t);
+      const float rest = a - hi;
+      h[e] = __float_as_uint(hi);
+      m[e] = __float_as_uint(rest);
+      l[e] = __float_as_uint(rest - __uint_as_float(m[e] & 0xFFFF0000u));
+    }
+    p.h[i] = pack_hi16(h[0], h[1]);
+    p.m[i] = pack_hi16(m[0], m[1]);
+    p.l[i] = pack_hi16(l[0], l[1]);
+    // (in asm: as C++ the ORs were put off to the end, with every l kept in a register)
+    asm volatile("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(l[0]), "v"(l[1]));
   }
   return p;
 }
@@ -126,7 +143,7 @@ __device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y, uint32_t& lost)
 // tile needs that (see above).
 template <bool KN, int BM, int BN, bool SPLITK, bool DMA16, bool EXACT>
 __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* smem) {
-  using S = F32Shape<BM, BN, DMA16>;
+  using S = F32Shape<BM, BN>;
   constexpr int FM = S::FM, FN = S::FN, NS = S::NS;
 
   const int tid = threadIdx.x;
@@ -153,7 +170,6 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
   // Row blocks: 4-byte instruction t writes slots 16 (t % 4) .. +15 of group t / 4, lane l
   // element l % 4 of slot 16 (t % 4) + l / 4.
   uint32_t a_off[S::A_DMA];
-  int a_k[S::A_DMA];
 #pragma unroll
   for (int i = 0; i < S::A_DMA; ++i) {
     const int t = wave * S::A_DMA + i;
@@ -162,13 +178,11 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
     const int row = 16 * (t >> 2) + r;
     const int k = 4 * c + (lane & 3);
     a_off[i] = (m0 + row < M) ? (uint32_t)(row * lda + k) * 4u : kBufOOB;
-    a_k[i] = k;
   }
   // B: [K,N] -> instruction t writes row k = t / (BN/64), floats 64*(t%(BN/64)) ..
   //    +63; lane l lands in segment slot 4*(t%(BN/64)) + l/16, which holds data
   //    segment slot ^ ((k/4)%4).  [N,K] -> as A.
   uint32_t b_off[S::B_DMA];
-  int b_k[S::B_DMA];
 #pragma unroll
   for (int i = 0; i < S::B_DMA; ++i) {
     const int t = wave * S::B_DMA + i;
@@ -178,14 +192,12 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
       const int seg = (4 * (t % PER_ROW) + (lane >> 4)) ^ ((k >> 2) & 3);
       const int n = 16 * seg + (lane & 15);
       b_off[i] = (n0 + n < N) ? (uint32_t)(k * ldb + n) * 4u : kBufOOB;
-      b_k[i] = k;
     } else {
       int r, c;
       f32_slot_src(16 * (t & 3) + (lane >> 2), r, c);
       const int row = 16 * (t >> 2) + r;
       const int k = 4 * c + (lane & 3);
       b_off[i] = (n0 + row < N) ? (uint32_t)(row * ldb + k) * 4u : kBufOOB;
-      b_k[i] = k;
     }
   }
   // DMA16 sources: A (and B as [N,K]) instruction t writes group t (rows 16t .. 16t+15),
@@ -257,12 +269,25 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
         for (int i = 0; i < S::B_DMA; ++i) dma_load4(rb, b_off[i], dst + S::A_BYTES + (wave * S::B_DMA + i) * 256);
         return;
       }
+      // each piece's k is found again here from an opaque copy of the lane: kept in registers
+      // over the loop, the ten of a 96 x 64 tile's were spilled (4097 x 3001 x 2049 370 -> 364 us)
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      auto row_k = [&](int t) {
+        int r, c;
+        f32_slot_src(16 * (t & 3) + (ln >> 2), r, c);
+        return 4 * c + (ln & 3);
+      };
 #pragma unroll
-      for (int i = 0; i < S::A_DMA; ++i)
-        dma_load4(ra, a_k[i] < krem ? a_off[i] : kBufOOB, dst + (wave * S::A_DMA + i) * 256);
+      for (int i = 0; i < S::A_DMA; ++i) {
+        const int t = wave * S::A_DMA + i;
+        dma_load4(ra, row_k(t) < krem ? a_off[i] : kBufOOB, dst + t * 256);
+      }
 #pragma unroll
-      for (int i = 0; i < S::B_DMA; ++i)
-        dma_load4(rb, b_k[i] < krem ? b_off[i] : kBufOOB, dst + S::A_BYTES + (wave * S::B_DMA + i) * 256);
+      for (int i = 0; i < S::B_DMA; ++i) {
+        const int t = wave * S::B_DMA + i;
+        dma_load4(rb, (KN ? t / (BN / 64) : row_k(t)) < krem ? b_off[i] : kBufOOB, dst + S::A_BYTES + t * 256);
+      }
     }
   };
 
@@ -274,6 +299,7 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
   const uint32_t fb_kn = S::A_BYTES + (uint32_t)(4 * g * BN * 4 + 4 * r16);
 
   f32x4 acc[FM][FN];
+  f32x4 small[FM][FN];  // the sums of the small products (not EXACT)
   // This wave's fragments of a stage (4 k per lane: k = 4g .. 4g+3)
   auto read_a = [&](int slot, int i) { return *(const f32x4*)(smem + slot * S::STAGE + fa + i * 1024); };
   auto read_b = [&](int slot, int j) {
@@ -286,37 +312,32 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
   };
 
   // Stages in ring slots slot and slot + 1 (32 k) on the bf16 instruction: B's next block is
-  // split while the current one's products run, the small products first.
+  // read and split while the current one's products run.
   uint32_t lost = 0;
   auto split_pair = [&](int slot) {
     F32Planes pa[FM], pb[FN];
-    f32x4 y0[FN], y1[FN];
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      y0[j] = read_b(slot, j);
-      y1[j] = read_b(slot + 1, j);
-    }
+    auto split_b = [&](int j) { pb[j] = f32_split(read_b(slot, j), read_b(slot + 1, j), lost); };
 #pragma unroll
     for (int i = 0; i < FM; ++i) pa[i] = f32_split(read_a(slot, i), read_a(slot + 1, i), lost);
-    pb[0] = f32_split(y0[0], y1[0], lost);
+    split_b(0);
     static_for<FN>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (j + 1 < FN) pb[j + 1] = f32_split(y0[j + 1], y1[j + 1], lost);
-      auto product = [&](u32x4 F32Planes::*b, u32x4 F32Planes::*a) {
+      if constexpr (j + 1 < FN) split_b(j + 1);
+      auto product = [&](f32x4(&sum)[FM][FN], u32x4 F32Planes::*b, u32x4 F32Planes::*a) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i) acc[i][j] = Mfma<__bf16>::mma(pb[j].*b, pa[i].*a, acc[i][j]);
+        for (int i = 0; i < FM; ++i) sum[i][j] = Mfma<__bf16>::mma(pb[j].*b, pa[i].*a, sum[i][j]);
       };
-      product(&F32Planes::l, &F32Planes::h);
-      product(&F32Planes::h, &F32Planes::l);
-      product(&F32Planes::m, &F32Planes::m);
-      product(&F32Planes::m, &F32Planes::h);
-      product(&F32Planes::h, &F32Planes::m);
-      product(&F32Planes::h, &F32Planes::h);
+      product(small, &F32Planes::l, &F32Planes::h);
+      product(small, &F32Planes::h, &F32Planes::l);
+      product(small, &F32Planes::m, &F32Planes::m);
+      product(small, &F32Planes::m, &F32Planes::h);
+      product(small, &F32Planes::h, &F32Planes::m);
+      product(acc, &F32Planes::h, &F32Planes::h);
       if constexpr (j + 1 < FN) {
         static_for<6 * FM>([&](auto) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one product,
-          __builtin_amdgcn_sched_group_barrier(0x002, (48 + 6 * FM - 1) / (6 * FM), 0);  // its share of the splitting
+          __builtin_amdgcn_sched_group_barrier(0x002, (56 + 6 * FM - 1) / (6 * FM), 0);  // its share of the splitting
         });
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -344,7 +365,7 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < FN; ++j) acc[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   load_stage(0);
   load_stage(1);
   certify();
@@ -365,9 +386,11 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < FN; ++j) {
+        acc[i][j] += small[i][j];
 #pragma unroll
         for (int e = 0; e < 4; ++e) again |= !(__builtin_fabsf(acc[i][j][e]) <= 3.402823466e+38f);
+      }
     // (through the ring, which is free: __syncthreads_or's own LDS would cost the 96 x 64 tile
     // its fourth workgroup per CU)
     uint32_t* any = (uint32_t*)smem;
@@ -449,7 +472,7 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
 // WAVES: waves per SIMD the kernel is compiled for (caps its registers at 512 / WAVES).
 template <bool KN, int BM, int BN, int WAVES, bool SPLITK = false, bool DMA16 = false>
 __global__ void __launch_bounds__(256, WAVES) gemm_f32_kernel(const GemmParams p) {
-  using S = F32Shape<BM, BN, DMA16>;
+  using S = F32Shape<BM, BN>;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[S::NS * S::STAGE];
   if (f32_tile<KN, BM, BN, SPLITK, DMA16, false>(p, smem)) f32_tile<KN, BM, BN, SPLITK, DMA16, true>(p, smem);
 }

@@ -1,7 +1,9 @@
 """The fp32 tiles that multiply on the bf16 matrix instruction (each float as three bf16
-planes, six products): single products to the last bits, infinities, NaN, the largest and
-the subnormal values as the fp32 instruction gives them, on every such tile, both B
-layouts, both loads (16- and 4-byte) and split K, against float64."""
+planes, six products): single products to the last bits, sums no further from the exact
+ones than a chain of fused multiply-adds, infinities, NaN, the largest and the subnormal
+values as the fp32 instruction gives them, on every such tile, both B layouts, both loads
+(16- and 4-byte) and split K, against float64."""
+import numpy as np
 import pytest
 import torch
 
@@ -24,16 +26,47 @@ def _run(monkeypatch, tile, a, b, nk, splits=1):
 @pytest.mark.parametrize("nk", [False, True])
 @pytest.mark.parametrize("M,N,K", [(130, 132, 4), (97, 65, 1), (128, 64, 33), (100, 200, 31)])
 def test_single_products(monkeypatch, tile, nk, M, N, K):
-    """One nonzero k: the result is one product, off by the three left-out plane products
-    (each below 2^-23 of it) and six roundings of 2^-24."""
+    """One nonzero k: the result is one product.  The left-out plane products come to at
+    most 2 * 2^-8 * 2^-16 of it, adding the two sums rounds by 2^-24, and the five small
+    products, 2^-7 of it, are added with a unit (2^-23) of their sum each."""
     g = torch.Generator().manual_seed(M + K)
     a, b = torch.zeros(M, K), torch.zeros(K, N)
     scale = lambda n: 2.0 ** torch.randint(-40, 41, (n,), generator=g)  # noqa: E731
-    a[:, K - 1] = (torch.rand(M, generator=g) + 1) * scale(M)
-    b[K - 1] = -(torch.rand(N, generator=g) + 1) * scale(N)
+    x, y = torch.rand(M, generator=g) + 1, -(torch.rand(N, generator=g) + 1)
+    for i, bits in enumerate([0x3F807FFF, 0x3F80FFFF, 0x3F808001, 0x3FFF7FFF, 0x3FFFFFFF, 0x3F800001]):
+        x[i] = y[i] = torch.tensor(bits, dtype=torch.int32).view(torch.float32)  # long rests
+    a[:, K - 1], b[K - 1] = x * scale(M), y * scale(N)
     out = _run(monkeypatch, tile, a.cuda(), b.cuda(), nk).double().cpu()
     exact = a[:, K - 1].double()[:, None] * b[K - 1].double()[None]
-    assert ((out - exact).abs() / exact.abs()).max().item() <= 3 * 2.0 ** -23 + 6 * 2.0 ** -24
+    assert ((out - exact).abs() / exact.abs()).max().item() <= 3 * 2.0 ** -24 + 5 * 2.0 ** -30
+
+
+def _chain(a, b):
+    """Each element as one chain of fused multiply-adds over k in fp32 (a product of two
+    floats is exact in float64, and rounding their sum twice moves a last bit in 2^29)."""
+    a, b = a.numpy().astype(np.float64), b.numpy().astype(np.float64)
+    c = np.zeros((a.shape[0], b.shape[1]), np.float32)
+    for k in range(a.shape[1]):
+        c = (c + a[:, k, None] * b[k]).astype(np.float32)
+    return c
+
+
+def _draw(kind, g, *shape):
+    x = torch.randn(shape, generator=g) if kind != "positive" else torch.rand(shape, generator=g)
+    return x.exp() if kind == "lognormal" else x
+
+
+@pytest.mark.parametrize("tile,nk", [(t, n) for t in TILES for n in (False, True)])
+@pytest.mark.parametrize("kind", ["normal", "positive", "lognormal"])
+def test_sums_against_a_chain(monkeypatch, tile, nk, kind):
+    for M, N, K in [(130, 68, 24), (96, 64, 100), (70, 65, 515), (130, 132, 2048), (64, 96, 8192)]:
+        g = torch.Generator().manual_seed(K)
+        a, b = _draw(kind, g, M, K), _draw(kind, g, K, N)
+        out = _run(monkeypatch, tile, a.cuda(), b.cuda(), nk).cpu().numpy().astype(np.float64)
+        exact = a.double().numpy() @ b.double().numpy()
+        err, chain = (np.linalg.norm(x - exact) / np.linalg.norm(exact) for x in (out, _chain(a, b)))
+        print(f"{tile} {kind} K={K}: {err:.2e}, a chain {chain:.2e}", flush=True)
+        assert err <= chain
 
 
 def _special(kind, M, N, K):
