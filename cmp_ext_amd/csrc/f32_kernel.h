@@ -81,37 +81,41 @@ __device__ __forceinline__ uint32_t f32_off(int row, int chunk) {
 }
 
 // ---- fp32 products on the bf16 matrix cores ----
-// A float x is the exact sum of three bf16 values: h, x rounded to 8 significant bits, m,
-// the top 8 bits of the signed rest, and l, what is left.  Of the nine products of two
-// such sums, six are summed in fp32 by v_mfma_f32_16x16x32_bf16: h h in one accumulator,
-// the five small ones (h m, m h, m m, h l, l h, in sum about 2^-7 of h h) in another, so
-// that they are rounded at their own size, and the two are added at the end.  (In one
-// accumulator the instruction cut the small products off below the sum's last bits,
-// always the same way: sums of 8192 positive products were off by 1.6e-5, the fp32
-// instruction's by 1.2e-6.)  m l, l m and l l are left out, together at most 2^-23 of the
-// product, and m's sign is independent of x's, so that they do not add up.  A chain
-// rounds once per 32 k where the fp32 instruction's (16x16x4) rounds 8 times.  Relative
-// Frobenius error against float64 on MI355X, fp32 instruction -> this: 512 x 512 x 8192
-// normal 1.62e-6 -> 0.57e-6, positive (uniform in [0, 1)) 1.19e-6 -> 0.42e-6, x 2048
-// 8.1e-7 -> 2.7e-7 and 6.0e-7 -> 2.2e-7, x 128 2.0e-7 -> 0.67e-7, x 32 1.0e-7 -> 0.41e-7,
-// x 16 7.4e-8 -> 3.6e-8, x 4 4.0e-8 -> 3.0e-8; x 1 2.5e-8 (one rounding) -> 3.0e-8, the
-// only one of these that is larger.
-// What the planes cannot hold -- infinities, floats of 2^112 and more (their m is a NaN) and
-// values with bits below bf16's smallest (under 2^-110 or so) -- is seen in the sums or in
-// l's dropped bits, and the tile is then computed again on the fp32 instruction.
-// Splitting an element takes 7 vector instructions in each wave that reads it, as many
+// A float x, taken as 2^16 x, is the exact sum of three bf16 values: h, 2^16 x rounded
+// to 8 significant bits, m, the top 8 bits of the signed rest, and l, what is left
+// (scaled, every bit of every float, subnormal ones too, is above bf16's smallest,
+// 2^-133).  Of the nine products of two such sums, six are summed in fp32 by
+// v_mfma_f32_16x16x32_bf16: h h in one accumulator, the five small ones (h m, m h, m m,
+// h l, l h, in sum about 2^-7 of h h) in another, so that they are rounded at their own
+// size, and the two are added at the end.  (In one accumulator the instruction cut the
+// small products off below the sum's last bits, always the same way: sums of 8192
+// positive products were off by 1.6e-5, the fp32 instruction's by 1.2e-6.)  m l, l m
+// and l l are left out, together at most 2^-23 of the product, and m's sign is
+// independent of x's, so that they do not add up.  A chain rounds once per 32 k where
+// the fp32 instruction's (16x16x4) rounds 8 times.  Relative Frobenius error against
+// float64 on MI355X, fp32 instruction -> this: 512 x 512 x 8192 normal 1.62e-6 ->
+// 0.57e-6, positive (uniform in [0, 1)) 1.19e-6 -> 0.42e-6, x 2048 8.1e-7 -> 2.7e-7 and
+// 6.0e-7 -> 2.2e-7, x 128 2.0e-7 -> 0.67e-7, x 32 1.0e-7 -> 0.41e-7, x 16 7.4e-8 ->
+// 3.6e-8, x 4 4.0e-8 -> 3.0e-8; x 1 2.5e-8 (one rounding) -> 3.0e-8, the only one of
+// these that is larger.
+// Infinities, NaN, floats of 2^96 and more and sums of 2^96 and more (their scaled values
+// overflow) are seen in the sums, and the tile is then computed again on the fp32
+// instruction: such a tile takes about 2.4 times as long as one that has none.
+// Splitting an element takes 6.5 vector instructions in each wave that reads it, as many
 // cycles as its products where a wave's block is small: that bounds the 96 x 64 and 64 x
 // 64 tiles (rounding by bf16 conversions took longer, 12 cycles each; one wave per K
 // stage, which splits less, left too few waves; sums of 32 k in registers of their own,
 // added to the total on the vector units, took 5 % longer than the two accumulators).
-// MI355X, fp32 instruction -> this: 4096^3 (128 x 128) 946 -> 760 us, 4097 x 3001 x 2049
-// (96 x 64, 4-byte DMA) 394 -> 396, 4100 x 3000 x 2048 (96 x 64) 369 -> 351, 3000 x 2000 x
-// 1000 (64 x 64) 101 -> 103.
+// MI355X, fp32 instruction -> this: 4096^3 (128 x 128) 946 -> 735 us, 4097 x 3001 x 2049
+// (96 x 64, 4-byte DMA) 394 -> 369, 4100 x 3000 x 2048 (96 x 64) 369 -> 336, 3000 x 2000 x
+// 1000 (64 x 64) 101 -> 98.
 struct F32Planes {
   u32x4 h, m, l;  // 8 k: two 16-k stages of 4
 };
-// The planes of eight floats; bits that bf16 drops from l go to `lost`.
-__device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y, uint32_t& lost) {
+constexpr float kF32Scale = 65536.f;                      // of a split float
+constexpr float kF32Unscale = 1.f / (65536.f * 65536.f);  // of a sum of products
+// The planes of eight floats.
+__device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y) {
   F32Planes p;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -120,10 +124,10 @@ __device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y, uint32_t& lost)
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const float a = v[2 * (i & 1) + e];
-      // t = 2^16 a + a to 24 bits, so t - 2^16 a is a to 8 bits, exactly, and so is the rest
-      const float t = a * 65537.f;
-      const float hi = __builtin_fmaf(a, -65536.f, t);
-      const float rest = a - hi;
+      // t = 2^32 a + 2^16 a to 24 bits, so t - 2^32 a is 2^16 a to 8 bits, exactly, and so is the rest
+      const float t = a * (kF32Scale * 65536.f + kF32Scale);
+      const float hi = __builtin_fmaf(a, -kF32Scale * 65536.f, t);
+      const float rest = __builtin_fmaf(a, kF32Scale, -hi);
       h[e] = __float_as_uint(hi);
       m[e] = __float_as_uint(rest);
       l[e] = __float_as_uint(rest - __uint_as_float(m[e] & 0xFFFF0000u));
@@ -131,8 +135,6 @@ __device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y, uint32_t& lost)
     p.h[i] = pack_hi16(h[0], h[1]);
     p.m[i] = pack_hi16(m[0], m[1]);
     p.l[i] = pack_hi16(l[0], l[1]);
-    // (in asm: as C++ the ORs were put off to the end, with every l kept in a register)
-    asm volatile("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(l[0]), "v"(l[1]));
   }
   return p;
 }
@@ -312,13 +314,13 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
   };
 
   // Stages in ring slots slot and slot + 1 (32 k) on the bf16 instruction: B's next block is
-  // read and split while the current one's products run.
-  uint32_t lost = 0;
+  // read and split among the current one's products (the fences between blocks only bound
+  // the registers; a fixed pattern of products and vector instructions was no faster).
   auto split_pair = [&](int slot) {
     F32Planes pa[FM], pb[FN];
-    auto split_b = [&](int j) { pb[j] = f32_split(read_b(slot, j), read_b(slot + 1, j), lost); };
+    auto split_b = [&](int j) { pb[j] = f32_split(read_b(slot, j), read_b(slot + 1, j)); };
 #pragma unroll
-    for (int i = 0; i < FM; ++i) pa[i] = f32_split(read_a(slot, i), read_a(slot + 1, i), lost);
+    for (int i = 0; i < FM; ++i) pa[i] = f32_split(read_a(slot, i), read_a(slot + 1, i));
     split_b(0);
     static_for<FN>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
@@ -334,12 +336,6 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
       product(small, &F32Planes::m, &F32Planes::h);
       product(small, &F32Planes::h, &F32Planes::m);
       product(acc, &F32Planes::h, &F32Planes::h);
-      if constexpr (j + 1 < FN) {
-        static_for<6 * FM>([&](auto) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one product,
-          __builtin_amdgcn_sched_group_barrier(0x002, (56 + 6 * FM - 1) / (6 * FM), 0);  // its share of the splitting
-        });
-      }
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -382,7 +378,7 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
     certify();
   }
   if constexpr (!EXACT) {
-    bool again = (lost & 0xFFFFu) != 0;
+    bool again = false;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -390,6 +386,7 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
         acc[i][j] += small[i][j];
 #pragma unroll
         for (int e = 0; e < 4; ++e) again |= !(__builtin_fabsf(acc[i][j][e]) <= 3.402823466e+38f);
+        acc[i][j] *= kF32Unscale;
       }
     // (through the ring, which is free: __syncthreads_or's own LDS would cost the 96 x 64 tile
     // its fourth workgroup per CU)

@@ -41,6 +41,38 @@ def test_single_products(monkeypatch, tile, nk, M, N, K):
     assert ((out - exact).abs() / exact.abs()).max().item() <= 3 * 2.0 ** -24 + 5 * 2.0 ** -30
 
 
+@pytest.mark.parametrize("tile,nk", [(t, n) for t in TILES for n in (False, True)])
+def test_single_products_of_tiny_floats(monkeypatch, tile, nk):
+    """Floats down to the smallest subnormal: no plane loses a bit (bounds as above; the
+    results, 2^-69 and more, are ordinary numbers)."""
+    M, N, K = 150, 68, 36
+    g = torch.Generator().manual_seed(1)
+    a, b = torch.zeros(M, K), torch.zeros(K, N)
+    a[:, K - 1] = (torch.rand(M, generator=g) + 1) * 2.0 ** torch.arange(-149, 1)
+    b[K - 1] = (torch.rand(N, generator=g) - 2) * 2.0 ** 80
+    assert (a[:, K - 1] > 0).all()
+    exact = a[:, K - 1].double()[:, None] * b[K - 1].double()[None]
+    for x, y, ref in ((a, b, exact), (b.t().contiguous(), a.t().contiguous(), exact.t())):
+        out = _run(monkeypatch, tile, x.cuda(), y.cuda(), nk).double().cpu()
+        assert ((out - ref).abs() / ref.abs()).max().item() <= 3 * 2.0 ** -24 + 5 * 2.0 ** -30
+
+
+@pytest.mark.parametrize("tile,nk", [(t, n) for t in TILES for n in (False, True)])
+@pytest.mark.parametrize("tiny", [1.2345e-35, 3e-39, 1.4e-45])
+def test_tiny_floats_stay_on_the_planes(monkeypatch, tile, nk, tiny):
+    """A tiny element does not send its tile to the fp32 instruction: every row and column
+    but its own has the bits that it has with a zero in its place."""
+    M, N, K = 130, 132, 200
+    g = torch.Generator().manual_seed(2)
+    a, b = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
+    a[7, 100] = b[33, 70] = 0.0
+    ref = _run(monkeypatch, tile, a.cuda(), b.cuda(), nk)
+    a[7, 100] = b[33, 70] = tiny
+    out = _run(monkeypatch, tile, a.cuda(), b.cuda(), nk)
+    rows, cols = torch.arange(M) != 7, torch.arange(N) != 70
+    assert torch.equal(out[rows][:, cols], ref[rows][:, cols])
+
+
 def _chain(a, b):
     """Each element as one chain of fused multiply-adds over k in fp32 (a product of two
     floats is exact in float64, and rounding their sum twice moves a last bit in 2^29)."""
