@@ -13,6 +13,10 @@ hipError_t launch(KernelId id, const GemmParams& p, dim3 grid, hipStream_t s) {
     case kF32Tile96x64:
       return launch_kernel((gemm_f32_kernel<KN, 96, 64, 4, SPLITK, DMA16>), grid, dim3(256), 0, s, p);
     case kF32Tile64:
+      if constexpr (!SPLITK) {
+        if (p.K <= kF32ShortK)
+          return launch_kernel((gemm_f32_short_kernel<KN, 64, 64, 8, DMA16>), grid, dim3(256), 0, s, p);
+      }
       return launch_kernel((gemm_f32_kernel<KN, 64, 64, 4, SPLITK, DMA16>), grid, dim3(256), 0, s, p);
     case kF32Tile64K4:
       return launch_kernel((gemm_f32_kwave_kernel<64, KN, 2, SPLITK, DMA16>), grid, dim3(256), 0, s, p);

@@ -17,6 +17,7 @@
 // address work.  The DMA fills a ring of four stages of BK = 16 k, two at a time
 // while the two before are multiplied; one wait and barrier per pair certifies that the
 // next pair has landed and that every wave is done with the slots about to be refilled.
+// Products of one stage (K <= 16) have a kernel of their own with one slot.
 //
 // LDS layouts (per stage):
 //   A, and B given as [N,K]: rows of 16 floats (64 bytes) in groups of 16 rows
@@ -38,10 +39,10 @@
 
 namespace cmpext3 {
 
-template <int BM, int BN>
+// NS: ring slots, four (two stages loaded and two multiplied at a time) or one (K <= BK).
+template <int BM, int BN, int NS>
 struct F32Shape {
   static constexpr int BK = 16;
-  static constexpr int NS = 4;    // ring slots, two stages loaded and two multiplied at a time
   static constexpr int NT = 256;  // 2 x 2 waves
   static constexpr int WTM = BM / 2, WTN = BN / 2;
   static constexpr int FM = WTM / 16, FN = WTN / 16;
@@ -96,9 +97,7 @@ __device__ __forceinline__ uint32_t f32_off(int row, int chunk) {
 // float64 on MI355X, fp32 instruction -> this: 512 x 512 x 8192 normal 1.62e-6 ->
 // 0.57e-6, positive (uniform in [0, 1)) 1.19e-6 -> 0.42e-6, x 2048 8.1e-7 -> 2.7e-7 and
 // 6.0e-7 -> 2.2e-7, x 128 2.0e-7 -> 0.67e-7, x 32 1.0e-7 -> 0.41e-7, x 16 7.4e-8 ->
-// 3.6e-8, x 4 4.0e-8 -> 3.0e-8; x 1 2.5e-8 (one rounding) -> 3.0e-8, the only one of
-// these that is larger.
-// Infinities, NaN, floats of 2^96 and more and sums of 2^96 and more (their scaled values
+// 3.6e-8, x 4 // Infinities, NaN, floats of 2^96 and more and sums of 2^96 and more (their scaled values
 // overflow) are seen in the sums, and the tile is then computed again on the fp32
 // instruction: such a tile takes about 2.4 times as long as one that has none.
 // Splitting an element takes 6.5 vector instructions in each wave that reads it, as many
@@ -142,11 +141,12 @@ __device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y) {
 // SPLITK: grid.z = batch * p.splits; this workgroup sums its split's K range and
 // stores the sums into p.partials (bias added by the reduction).
 // EXACT: on the fp32 instruction.  Otherwise returns true, with nothing written, when the
-// tile needs that (see above).
-template <bool KN, int BM, int BN, bool SPLITK, bool DMA16, bool EXACT>
+// tile needs that (see above).  NS: ring slots; one for K <= 16 (EXACT).
+template <bool KN, int BM, int BN, bool SPLITK, bool DMA16, bool EXACT, int NS = 4>
 __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* smem) {
-  using S = F32Shape<BM, BN>;
-  constexpr int FM = S::FM, FN = S::FN, NS = S::NS;
+  using S = F32Shape<BM, BN, NS>;
+  constexpr int FM = S::FM, FN = S::FN;
+  static_assert(NS == 4 || (NS == 1 && EXACT && !SPLITK), "a ring of four stages, or one stage");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -355,27 +355,32 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
   // every load has landed and every wave's reads are done
   auto certify = [&]() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
 
-  // Two stages at a time: stages st+2 and st+3 (zeros past K) load into the slots that the
-  // iteration before read while st and st+1 are multiplied.
-  const int nst = (K + S::BK - 1) / S::BK;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   load_stage(0);
-  load_stage(1);
-  certify();
-  for (int st = 0; st < nst; st += 2) {
-    const int slot = st & 2;
-    load_stage(st + 2);
-    load_stage(st + 3);
-    if constexpr (EXACT) {
-      exact_stage(slot);
-      exact_stage(slot + 1);
-    } else {
-      split_pair(slot);
-    }
+  if constexpr (NS == 1) {
     certify();
+    exact_stage(0);
+  } else {
+    // Two stages at a time: stages st+2 and st+3 (zeros past K) load into the slots that the
+    // iteration before read while st and st+1 are multiplied.
+    const int nst = (K + S::BK - 1) / S::BK;
+    load_stage(1);
+    certify();
+    for (int st = 0; st < nst; st += 2) {
+      const int slot = st & 2;
+      load_stage(st + 2);
+      load_stage(st + 3);
+      if constexpr (EXACT) {
+        exact_stage(slot);
+        exact_stage(slot + 1);
+      } else {
+        split_pair(slot);
+      }
+      certify();
+    }
   }
   if constexpr (!EXACT) {
     bool again = false;
@@ -469,9 +474,23 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
 // WAVES: waves per SIMD the kernel is compiled for (caps its registers at 512 / WAVES).
 template <bool KN, int BM, int BN, int WAVES, bool SPLITK = false, bool DMA16 = false>
 __global__ void __launch_bounds__(256, WAVES) gemm_f32_kernel(const GemmParams p) {
-  using S = F32Shape<BM, BN>;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[S::NS * S::STAGE];
-  if (f32_tile<KN, BM, BN, SPLITK, DMA16, false>(p, smem)) f32_tile<KN, BM, BN, SPLITK, DMA16, true>(p, smem);
+  using S = F32Shape<BM, BN, 4>;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * S::STAGE];
+  if (p.K <= kF32ShortK || f32_tile<KN, BM, BN, SPLITK, DMA16, false>(p, smem))
+    f32_tile<KN, BM, BN, SPLITK, DMA16, true>(p, smem);
+}
+
+// K <= kF32ShortK: products of one stage are bound by writing C, and each sum has too few
+// terms for the planes to round it less often than the fp32 instruction does.  One load and
+// no ring, so that eight workgroups share a CU and some write their tiles while others wait
+// for their operands.  MI355X, 64 x 64 tiles, the ring kernel on planes -> this: 4096 x 4096
+// x 16 22.4 -> 15.9 us (4.2 TB/s written), 8192 x 1024 x 8 13.7 -> 10.3, 3000 x 2001 x 1 (rows
+// not 16-byte aligned) 20.4 -> 18.0, 1000 x 1001 x 16 6.8 -> 5.7.
+template <bool KN, int BM, int BN, int WAVES, bool DMA16>
+__global__ void __launch_bounds__(256, WAVES) gemm_f32_short_kernel(const GemmParams p) {
+  using S = F32Shape<BM, BN, 1>;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[S::STAGE];
+  f32_tile<KN, BM, BN, false, DMA16, true, 1>(p, smem);
 }
 
 }  // namespace cmpext3

@@ -30,6 +30,9 @@ struct GemmParams {
   float* partials;
 };
 
+// fp32 products of at most this many k run on the fp32 instruction (f32_kernel.h).
+constexpr int kF32ShortK = 16;
+
 // Every kernel the library can launch.  The selector returns one of these.
 enum KernelId : int {
   kTile256x256 = 0,   // f16/bf16 MFMA 16x16x32, 8 waves of 64x128, LDS-DMA ring

@@ -371,6 +371,11 @@ int make_plan_core(const Request& r, Plan* plan) {
     double best_cost = -1.0;
     for (const F32Tile& c : kTiles32) {
       if (c.bm == 16 && r.M > 16) continue;  // 16-row tiles: measured and meant for M <= 16 only
+      // K <= 16 is bound by writing C: 64x64 tiles, eight to a CU (gemm_f32_short_kernel), were
+      // the fastest of all tiles at each of 15 outputs from 64 x 64 to 100000 x 16 and K = 1 ..
+      // 16 (MI355X, against the fastest other: 4096 x 4096 x 16 15.9 and 22.1 us, 2048 x 2048 x 4
+      // 7.4 and 9.4, 16 x 100000 x 16 7.5 and 7.3 with 16x64k4, the one it loses, by 3 %)
+      if (r.K <= kF32ShortK && c.id != kF32Tile64) continue;
       const int64_t smax = (r.N % 4 == 0 && r.K >= 1024) ? std::min<int64_t>(16, r.K / 256) : 1;
       for (int64_t s = 1; s <= std::max<int64_t>(1, smax); ++s) {
         if (s > 1 && s * r.batch * r.M * r.N * 4 > r.ws_bytes) break;

@@ -101,6 +101,48 @@ def test_sums_against_a_chain(monkeypatch, tile, nk, kind):
         assert err <= chain
 
 
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("K", [1, 3, 16])
+def test_short_sums_keep_the_fp32_instruction(monkeypatch, tile, nk, K):
+    """K <= 16: one product is rounded once, on every tile."""
+    g = torch.Generator().manual_seed(K)
+    a, b = torch.zeros(130, K), torch.zeros(K, 132)
+    a[:, K - 1], b[K - 1] = torch.randn(130, generator=g), torch.randn(132, generator=g)
+    out = _run(monkeypatch, tile, a.cuda(), b.cuda(), nk).cpu()
+    assert torch.equal(out, a[:, K - 1, None] * b[K - 1])
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (63, 64), (64, 65), (129, 200), (1000, 1001), (4, 3000)])
+@pytest.mark.parametrize("K", [0, 1, 2, 4, 15, 16, 17, 31, 32, 33])
+@pytest.mark.parametrize("nk", [False, True])
+def test_short_k(M, N, K, nk):
+    """The kernel for one stage and the first sizes past it, with a bias: no element further
+    off than K + 1 roundings of its terms."""
+    g = torch.Generator().manual_seed(M + K)
+    x, w, bias = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g), torch.randn(N, generator=g)
+    if nk:
+        out = cmpext3.linear(x.cuda(), w.cuda(), bias.cuda())
+    else:
+        out, bias = cmpext3.fp32_matmul(x.cuda(), w.t().contiguous().cuda()), torch.zeros(N)
+    desc = cmpext3.last_plan()
+    print(M, N, K, desc, flush=True)
+    assert K > 16 or desc.startswith("kernel=f32tile64x64 ")
+    x, w, bias = x.double(), w.double(), bias.double()
+    err = (out.double().cpu() - (x @ w.t() + bias)).abs()
+    assert (err <= (K + 1) * 2.0 ** -24 * (x.abs() @ w.abs().t() + bias.abs())).all()
+
+
+def test_short_k_batches():
+    g = torch.Generator().manual_seed(0)
+    for B, M, N, K in [(3, 65, 70, 16), (2, 100, 33, 7), (5, 1, 64, 16)]:
+        a, b = torch.randn(B, M, K, generator=g), torch.randn(B, K, N, generator=g)
+        out = cmpext3.bmm(a.cuda(), b.cuda()).double().cpu()
+        for i in range(B):
+            size = a[i].double().abs() @ b[i].double().abs()
+            assert ((out[i] - a[i].double() @ b[i].double()).abs() <= K * 2.0 ** -24 * size).all()
+
+
 def _special(kind, M, N, K):
     g = torch.Generator().manual_seed(7)
     a, b = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
