@@ -105,24 +105,24 @@ __device__ __forceinline__ uint32_t f32_off(int row, int chunk) {
 // 64 tiles (rounding by bf16 conversions took longer, 12 cycles each; one wave per K
 // stage, which splits less, left too few waves; sums of 32 k in registers of their own,
 // added to the total on the vector units, took 5 % longer than the two accumulators).
-// MI355X, fp32 instruction -> this: 4096^3 (128 x 128) 946 -> 735 us, 4097 x 3001 x 2049
-// (96 x 64, 4-byte DMA) 394 -> 369, 4100 x 3000 x 2048 (96 x 64) 369 -> 336, 3000 x 2000 x
-// 1000 (64 x 64) 101 -> 98.
-struct F32Planes {
-  u32x4 h, m, l;  // 8 k: two 16-k stages of 4
-};
+// MI355X, fp32 instruction -> this: 4096^3 (128 x 128) 946 -> 732 us, 4097 x 3001 x 2049
+// (96 x 64, 4-byte DMA) 394 -> 362, 4100 x 3000 x 2048 (96 x 64) 369 -> 333, 3000 x 2000 x
+// 1000 (64 x 64) 101 -> 97.
 constexpr float kF32Scale = 65536.f;                      // of a split float
 constexpr float kF32Unscale = 1.f / (65536.f * 65536.f);  // of a sum of products
-// The planes of eight floats.
-__device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y) {
-  F32Planes p;
+template <typename V>
+struct F32Planes {
+  V h, m, l;  // u32x4: 8 k, two 16-k stages of 4; u32x2: one stage's 4
+};
+// Words i, i+1 of the planes of four floats.
+template <typename V>
+__device__ __forceinline__ void f32_split4(F32Planes<V>& p, int i, f32x4 x) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const f32x4 v = i < 2 ? x : y;
+  for (int w = 0; w < 2; ++w) {
     uint32_t h[2], m[2], l[2];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      const float a = v[2 * (i & 1) + e];
+      const float a = x[2 * w + e];
       // t = 2^32 a + 2^16 a to 24 bits, so t - 2^32 a is 2^16 a to 8 bits, exactly, and so is the rest
       const float t = a * (kF32Scale * 65536.f + kF32Scale);
       const float hi = __builtin_fmaf(a, -kF32Scale * 65536.f, t);
@@ -131,11 +131,15 @@ __device__ __forceinline__ F32Planes f32_split(f32x4 x, f32x4 y) {
       m[e] = __float_as_uint(rest);
       l[e] = __float_as_uint(rest - __uint_as_float(m[e] & 0xFFFF0000u));
     }
-    p.h[i] = pack_hi16(h[0], h[1]);
-    p.m[i] = pack_hi16(m[0], m[1]);
-    p.l[i] = pack_hi16(l[0], l[1]);
+    p.h[i + w] = pack_hi16(h[0], h[1]);
+    p.m[i + w] = pack_hi16(m[0], m[1]);
+    p.l[i + w] = pack_hi16(l[0], l[1]);
   }
-  return p;
+}
+__device__ __forceinline__ f32x4 f32_mma(u32x4 b, u32x4 a, f32x4 c) { return Mfma<__bf16>::mma(b, a, c); }
+__device__ __forceinline__ f32x4 f32_mma(u32x2 b, u32x2 a, f32x4 c) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, b), __builtin_bit_cast(s16x4, a), c, 0, 0, 0);
 }
 
 // SPLITK: grid.z = batch * p.splits; this workgroup sums its split's K range and
@@ -313,29 +317,40 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
     return x;
   };
 
-  // Stages in ring slots slot and slot + 1 (32 k) on the bf16 instruction: B's next block is
-  // read and split among the current one's products (the fences between blocks only bound
-  // the registers; a fixed pattern of products and vector instructions was no faster).
-  auto split_pair = [&](int slot) {
-    F32Planes pa[FM], pb[FN];
-    auto split_b = [&](int j) { pb[j] = f32_split(read_b(slot, j), read_b(slot + 1, j)); };
+  // The stages in ring slots slot and slot + 1 (V = u32x4: 32 k), or the one in slot (u32x2:
+  // 16 k), on the bf16 instruction: B's next block is read and split among the current
+  // one's products (the fences between blocks only bound the registers; a fixed pattern of
+  // products and vector instructions was no faster).
+  auto split_stages = [&](int slot, auto v) {
+    using V = decltype(v);
+    using P = F32Planes<V>;
+    constexpr bool PAIR = sizeof(V) == sizeof(u32x4);
+    P pa[FM], pb[FN];
+    auto split_a = [&](int i) {
+      f32_split4(pa[i], 0, read_a(slot, i));
+      if constexpr (PAIR) f32_split4(pa[i], 2, read_a(slot + 1, i));
+    };
+    auto split_b = [&](int j) {
+      f32_split4(pb[j], 0, read_b(slot, j));
+      if constexpr (PAIR) f32_split4(pb[j], 2, read_b(slot + 1, j));
+    };
 #pragma unroll
-    for (int i = 0; i < FM; ++i) pa[i] = f32_split(read_a(slot, i), read_a(slot + 1, i));
+    for (int i = 0; i < FM; ++i) split_a(i);
     split_b(0);
     static_for<FN>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (j + 1 < FN) split_b(j + 1);
-      auto product = [&](f32x4(&sum)[FM][FN], u32x4 F32Planes::*b, u32x4 F32Planes::*a) {
+      auto product = [&](f32x4(&sum)[FM][FN], V P::*b, V P::*a) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i) sum[i][j] = Mfma<__bf16>::mma(pb[j].*b, pa[i].*a, sum[i][j]);
+        for (int i = 0; i < FM; ++i) sum[i][j] = f32_mma(pb[j].*b, pa[i].*a, sum[i][j]);
       };
-      product(small, &F32Planes::l, &F32Planes::h);
-      product(small, &F32Planes::h, &F32Planes::l);
-      product(small, &F32Planes::m, &F32Planes::m);
-      product(small, &F32Planes::m, &F32Planes::h);
-      product(small, &F32Planes::h, &F32Planes::m);
-      product(acc, &F32Planes::h, &F32Planes::h);
+      product(small, &P::l, &P::h);
+      product(small, &P::h, &P::l);
+      product(small, &P::m, &P::m);
+      product(small, &P::m, &P::h);
+      product(small, &P::h, &P::m);
+      product(acc, &P::h, &P::h);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -359,26 +374,40 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  load_stage(0);
   if constexpr (NS == 1) {
+    load_stage(0);
     certify();
     exact_stage(0);
   } else {
-    // Two stages at a time: stages st+2 and st+3 (zeros past K) load into the slots that the
-    // iteration before read while st and st+1 are multiplied.
+    // Two stages at a time: stages st+2 and st+3 load into the slots that the iteration
+    // before read while st and st+1 are multiplied.  Nothing is loaded past K, and an odd
+    // stage is multiplied alone, by 16x16x16 products (a stage of zeros beside it took as
+    // long as a full one: 20000 x 256 x 40 12.7 -> 11.5 us, 4096 x 4096 x 40 26.1 -> 24.3,
+    // 1000 x 1001 x 24 7.5 -> 7.1).
     const int nst = (K + S::BK - 1) / S::BK;
-    load_stage(1);
+    auto load_pair = [&](int st) {
+      if (st < nst) load_stage(st);
+      if (st + 1 < nst) load_stage(st + 1);
+    };
+    load_pair(0);
     certify();
-    for (int st = 0; st < nst; st += 2) {
+    for (int st = 0; st + 1 < nst; st += 2) {
       const int slot = st & 2;
-      load_stage(st + 2);
-      load_stage(st + 3);
+      load_pair(st + 2);
       if constexpr (EXACT) {
         exact_stage(slot);
         exact_stage(slot + 1);
       } else {
-        split_pair(slot);
+        split_stages(slot, u32x4{});
       }
+      certify();
+    }
+    if (nst > 0 && (nst & 1)) {  // the last stage alone (a split past K's end has none)
+      const int slot = (nst - 1) & 2;
+      if constexpr (EXACT)
+        exact_stage(slot);
+      else
+        split_stages(slot, u32x2{});
       certify();
     }
   }

@@ -143,6 +143,22 @@ def test_short_k_batches():
             assert ((out[i] - a[i].double() @ b[i].double()).abs() <= K * 2.0 ** -24 * size).all()
 
 
+@pytest.mark.parametrize("M,N,K,nk", [(198, 896, 5976, True), (512, 512, 4096, False), (329, 392, 8002, True),
+                                      (23, 2236, 8230, True), (656, 140, 7368, False)])
+def test_splits_past_the_end_of_k(M, N, K, nk):
+    """Splits are whole numbers of 64 k, so the last may start past K: it adds zeros."""
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    torch.full((1 << 24,), float("nan"), device="cuda")  # (what the workspace may have held)
+    out = cmpext3.linear(x.cuda(), w.cuda()) if nk else cmpext3.fp32_matmul(x.cuda(), w.t().contiguous().cuda())
+    desc = cmpext3.last_plan()
+    print(M, N, K, desc, flush=True)
+    assert "splits=" in desc
+    ref = (x.double() @ w.double().t()).numpy()
+    # K / 32 roundings of the partial sums, and one for each split
+    assert np.linalg.norm(out.double().cpu().numpy() - ref) <= 1e-6 * np.linalg.norm(ref)
+
+
 def _special(kind, M, N, K):
     g = torch.Generator().manual_seed(7)
     a, b = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)

@@ -396,3 +396,9 @@ def test_row_split_plans_cover_the_rows():
         if ws == 0:
             assert "workspace=" not in desc, desc
     assert splits >= 10
+
+
+@pytest.mark.parametrize("M,N,K", [(1024, 1024, 24), (1000, 1001, 32), (256, 256, 17), (128, 2048, 32)])
+def test_fp32_tile_of_two_stages(M, N, K):
+    """17 to 32 k leave half of 64x64k4's waves without a stage."""
+    assert "kernel=f32tile64x64 " in cabi.plan(cabi.F32, cabi.B_KN, M, N, K)[1]
