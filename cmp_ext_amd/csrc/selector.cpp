@@ -63,32 +63,37 @@ const Candidate kTiles16[] = {
 // workgroup, latency-bound) to umax (occ of them and more), in units of the fp32
 // instruction's rate, which 128x128, 96x64 and 64x64 can exceed (they run on the bf16
 // instruction, f32_kernel.h).  Their numbers follow timings of every tile with 1, 2, 3,
-// 4 and 8 K splits on 15 shapes (MI355X; M 64..4097, N 1000..4096, K 500..8192): 128x128,
-// whose waves split the fewest operand elements per product, 1.0 alone and 1.09..1.25 in
-// pairs, 96x64 0.65 alone and 0.93..0.98 with four to eight, 64x64 0.45..0.55 and
-// 0.84..0.89.  Its choices against the ones before, on the same kernels: 512 x 4096 x 4096
-// 139.5 -> 106.7 us (128x128 in 4 splits for 64x64 in 4), 2048^3 136 -> 104, 384 columns
-// x[1997, 3840] 60 -> 47.7.  The 4-byte LDS-DMA path (rows not 16-byte aligned) scales
-// umax by dma4.  64x64k4 (K split over the four waves, two workgroups per CU; fp32
-// instruction) was fitted to 114 timings: u1 0.62, umax 0.72; 16x64k4 (M <= 16, bound by
-// streaming B) to 134 more over 29 shapes with M <= 16: u1 0.36, umax 0.46, and a CU
-// streams its workgroups' B strips at ~19 GB/s with one of them, ~24 GB/s with more
-// (6 TB/s over 256 CUs).  64x64k4's lead is its waves' sums being added up: without it 17
-// to 32 k, where half its waves have no stage, were planned on it (1024 x 1024 x 32 5.7 us,
-// 64x64 5.0).
+// 4 and 8 K splits on 15 shapes (MI355X; M 64..4097, N 1000..4096, K 500..8192):
+// 128x128, whose waves split the fewest operand elements per product, 1.0 alone and
+// 1.09..1.25 in pairs, 96x64 0.65 alone and 0.93..0.98 with four to eight, 64x64
+// 0.45..0.55 and 0.84..0.89.  Its choices against the ones before, on the same kernels:
+// 512 x 4096 x 4096 139.5 -> 106.7 us (128x128 in 4 splits for 64x64 in 4), 2048^3 136
+// -> 104, 384 columns x[1997, 3840] 60 -> 47.7.  The 4-byte LDS-DMA path (rows not
+// 16-byte aligned) scales umax by dma4, and what a tile alone on its CU reaches by
+// lone4: 128x128 tiles whose K cannot be split (N % 4 != 0) were taken at the aligned
+// rate, 3435 x 731 x 7226 505 us for 64x64 tiles' 376, 1677 x 1661 x 8195 567 for 421
+// (MI355X; of 98 drawn products whose choice it changes 90 gain up to 22 %, eight lose
+// 5 to 15 %).  64x64k4 (K split over the four waves, two workgroups per CU; fp32
+// instruction) was fitted to 114 timings: u1 0.62, umax 0.72; 16x64k4 (M <= 16, bound
+// by streaming B) to 134 more over 29 shapes with M <= 16: u1 0.36, umax 0.46, and a CU
+// streams its workgroups' B strips at ~19 GB/s with one of them, ~24 GB/s with more (6
+// TB/s over 256 CUs).  64x64k4's lead is its waves' sums being added up: without it 17
+// to 32 k, where half its waves have no stage, were planned on it (1024 x 1024 x 32 5.7
+// us, 64x64 5.0).
 struct F32Tile {
   KernelId id;
   int bm, bn, occ;
-  double u1, umax, dma4;
+  double u1, umax;
+  double lone4, dma4;  // of u1 alone on a CU, of umax otherwise, on the 4-byte path
   int kwaves;  // waves that split a workgroup's 16-k steps among them
   int lead;    // steps that filling its ring and storing its tile cost a CU's last one
 };
 const F32Tile kTiles32[] = {
-    {kF32Tile128, 128, 128, 2, 0.95, 1.14, 0.82, 1, 2},
-    {kF32Tile96x64, 96, 64, 8, 0.655, 0.95, 0.975, 1, 1},
-    {kF32Tile64, 64, 64, 3, 0.45, 0.845, 0.84, 1, 1},
-    {kF32Tile64K4, 64, 64, 2, 0.62, 0.72, 0.84, 4, 1},
-    {kF32Tile16K4, 16, 64, 4, 0.36, 0.46, 0.84, 4, 4},
+    {kF32Tile128, 128, 128, 2, 0.95, 1.14, 0.79, 0.82, 1, 2},
+    {kF32Tile96x64, 96, 64, 8, 0.655, 0.95, 0.80, 0.975, 1, 1},
+    {kF32Tile64, 64, 64, 3, 0.45, 0.845, 0.91, 0.84, 1, 1},
+    {kF32Tile64K4, 64, 64, 2, 0.62, 0.72, 0.90, 0.84, 4, 1},
+    {kF32Tile16K4, 16, 64, 4, 0.36, 0.46, 1.00, 0.84, 4, 4},
 };
 // Modelled microseconds: w = workgroups on the busiest CU, each running cdiv(K/s, 16)
 // steps of bm*bn*16 MFMA work (bm*bn*32 / (256 * 2380) us at the full fp32 rate of a
@@ -100,7 +105,8 @@ double f32_cost(const F32Tile& c, int64_t M, int64_t N, int64_t K, int64_t batch
   const double steps = (double)(cdiv(cdiv(cdiv(K, s), 16), c.kwaves) * c.kwaves);
   const double step_us = c.bm * c.bn * 32.0 / (256.0 * 2380.0);
   const double umax = dma16 ? c.umax : c.dma4 * c.umax;
-  const double u = c.u1 + (umax - c.u1) * std::min(1.0, (double)(w - 1) / (c.occ - 1));
+  double u = c.u1 + (umax - c.u1) * std::min(1.0, (double)(w - 1) / (c.occ - 1));
+  if (w == 1 && !dma16) u *= c.lone4;
   const double mem = std::max((double)batch * (M * K + K * N) * 4.0 / 5.4e6,
                               (double)w * c.bn * cdiv(K, s) * 4.0 / (w == 1 ? 19e3 : 24e3));
   double t = 1.0 + std::max(((double)w * steps + c.lead) * step_us / u, mem);

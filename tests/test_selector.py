@@ -402,3 +402,9 @@ def test_row_split_plans_cover_the_rows():
 def test_fp32_tile_of_two_stages(M, N, K):
     """17 to 32 k leave half of 64x64k4's waves without a stage."""
     assert "kernel=f32tile64x64 " in cabi.plan(cabi.F32, cabi.B_KN, M, N, K)[1]
+
+
+@pytest.mark.parametrize("M,N,K,nk", [(3435, 731, 7226, True), (1677, 1661, 8195, True), (2109, 1415, 7975, False)])
+def test_fp32_lone_tiles_on_4_byte_rows(M, N, K, nk):
+    """One 128x128 tile per CU and a K that cannot be split: slower than more, smaller tiles."""
+    assert "kernel=f32tile64x64 " in cabi.plan(cabi.F32, cabi.B_NK if nk else cabi.B_KN, M, N, K)[1]
