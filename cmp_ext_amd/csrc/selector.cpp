@@ -446,7 +446,9 @@ int make_plan_core(const Request& r, Plan* plan) {
       // strips (x[64, 4096] W[14336, 4096]^T) 2 ways took 39.2 us against 29.3.
       p = skinny_nk_plan(r, 1, p.group_m);
       const int64_t chunk = std::min<int64_t>(r.batch, 65535);
-      const int64_t wgs = cdiv(r.N, p.bn) * chunk, wgs64 = cdiv(r.N, 64) * chunk;
+      // (empty products -- N or batch 0 -- launch nothing; keep the arithmetic defined)
+      const int64_t wgs = std::max<int64_t>(1, cdiv(r.N, p.bn) * chunk);
+      const int64_t wgs64 = std::max<int64_t>(1, cdiv(r.N, 64) * chunk);
       if (2 * wgs <= kNumCUs && (int64_t)(p.bn + p.bm) * r.K * 2 >= 700000) {
         p = skinny_nk_plan(r, std::min<int64_t>(8, std::max<int64_t>(2, kNumCUs / wgs)), p.group_m);
       } else if (p.mb >= 2 && r.K >= 10240 && 2 * wgs64 <= kNumCUs) {
@@ -520,7 +522,8 @@ int make_plan_core(const Request& r, Plan* plan) {
       // workgroups run (fp32 partials, a second launch sums them; MI355X, fp16, vs the
       // selector's tile128x128 split 16 ways: 1024 x 16 x 14336 9.9 vs 14.3 us, 1024 x 64 x
       // 14336 13.0 vs 15.5, 2048 x 8 x 14336 13.3 vs 16.4, 1024 x 64 x 8192 10.7 vs 11.6)
-      p = tall_plan(r, 32, p.group_m, std::min<int64_t>(8, kNumCUs / (cdiv(r.M, 32) * r.batch)));
+      p = tall_plan(r, 32, p.group_m,
+                    std::min<int64_t>(8, kNumCUs / std::max<int64_t>(1, cdiv(r.M, 32) * r.batch)));
     } else if (fast && r.M <= 64 && r.K <= 1024 && cdiv(r.N, 256) * r.batch >= kNumCUs) {
       // Short-K products with few rows and many columns are HBM-bound; 64-row tiles
       // waste no MFMA rows and keep more loads in flight per CU (MI355X, 64x256 vs

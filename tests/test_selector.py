@@ -1,4 +1,6 @@
 """Host-side kernel selection and argument validation (no GPU needed)."""
+import itertools
+
 import pytest
 
 from cmp_ext_amd import cabi
@@ -217,6 +219,18 @@ def test_zero_sizes_are_valid():
     for M, N, K in [(0, 5, 5), (5, 0, 5), (5, 5, 0)]:
         kid, _ = cabi.plan(cabi.F16, cabi.B_KN, M, N, K)
         assert kid >= 0
+
+
+def test_empty_products_of_every_kernel_plan():
+    """No rows, columns, k or batch entries, with the other sizes those of every rule that
+    divides by a number of workgroups."""
+    sizes = [0, 1, 16, 33, 64, 128, 2048, 14336]
+    for dtype in (cabi.F16, cabi.F32):
+        for layout in (cabi.B_KN, cabi.B_NK):
+            for M, N, K, batch in itertools.product(sizes, sizes, sizes, (0, 1, 3)):
+                if 0 in (M, N, K, batch):
+                    assert cabi.plan(dtype, layout, M, N, K, batch=batch, workspace_bytes=1 << 40)[0] >= 0
+                    assert cabi.workspace_size(dtype, layout, M, N, K, batch) >= 0
 
 
 @pytest.mark.parametrize("layout,M,N,K,batch,expect,strip", [

@@ -70,3 +70,13 @@ def test_strips_of_a_batch_and_of_whole_layers():
         assert desc.startswith("kernel=skinny_nk") and f"x{strip} " in desc, desc
         for i in range(batch):
             assert O.reference_check(out[i].cpu(), x[i], w[i], "fp16", None, "NK") <= O.TOLERANCE["fp16"]
+
+
+@pytest.mark.gpu
+def test_linear_without_rows_or_outputs():
+    import cmpext3
+
+    x, w = torch.randn(16, 14336).half().cuda(), torch.randn(8, 14336).half().cuda()
+    assert cmpext3.linear(x, w[:0]).shape == (16, 0)
+    assert cmpext3.linear(x[:0], w).shape == (0, 8)
+    assert cmpext3.bmm(x[None][:0], w.t()[None][:0]).shape == (0, 16, 8)
