@@ -406,9 +406,15 @@ int make_plan_core(const Request& r, Plan* plan) {
     }
     override32(r, dma16, &p);
   } else {
-    const bool skinny_ok = r.M <= 64 && r.align >= 16 && r.K % 8 == 0 &&
-                           r.lda % 8 == 0 && r.N % 8 == 0 && r.ldb % 8 == 0 &&
-                           (!batched || (r.stride_a % 8 == 0 && r.stride_b % 8 == 0));
+    // (r.b_dword: r.align speaks of A and C, B's rows and its address are aligned to 4 bytes.
+    // The skinny kernels take such a B as the tile kernels do, by 16-byte LDS-DMA pieces from
+    // 4-byte aligned sources; with N % 8 == 0 no piece crosses a row's end.  MI355X, fp16, B's
+    // rows 4 bytes longer than N, padded copy and skinny_wide -> in place (a 128x128 tile
+    // in place): 16 x 4096 x 4096 23.5 -> 11.1 us (40.1), 16 x 512 x 8192 20.1 -> 9.8 (75.7),
+    // 8 x 4096 x 14336 62.6 -> 21.0 (131), 32 x 14336 x 4096 66.2 -> 31.5 (40.9).)
+    const bool skinny_ok = r.M <= 64 && r.align >= 16 && r.K % 8 == 0 && r.lda % 8 == 0 && r.N % 8 == 0 &&
+                           (r.ldb % 8 == 0 || r.b_dword) &&
+                           (!batched || (r.stride_a % 8 == 0 && (r.stride_b % 8 == 0 || r.b_dword)));
     // (the tiled kernels' epilogue stores in 16-, 8- or 2-byte pieces as C's rows allow)
     const bool fast = r.align >= 16 && r.K % 8 == 0 && r.lda % 8 == 0 && (r.ldb % 8 == 0 || r.b_dword) &&
                       (r.layout == kNK || r.N % 8 == 0 || r.b_cols_padded || r.b_dword) &&

@@ -1,7 +1,7 @@
 """16-bit products whose B is [K, N] with rows aligned to 4 bytes only (an even N or pitch
-that is no multiple of 8: images of 14x14 pixels) are read in place by the tile kernels:
-which calls take that route (CPU), and its results, with NaN after every row and after the
-operand, against the float64 oracle."""
+that is no multiple of 8: images of 14x14 pixels) are read in place by the tile kernels and,
+for at most 64 rows and N % 8 == 0, the skinny ones: which calls take that route (CPU), and
+its results, with NaN after every row and after the operand, against the float64 oracle."""
 import numpy as np
 import pytest
 import torch
@@ -34,13 +34,18 @@ def test_route():
         aligned_b = off_b % 8 == 0 and ldb % 8 == 0 and N % 8 == 0
         even = off_b % 2 == 0 and ldb % 2 == 0 and (batch == 1 or K * ldb % 2 == 0)
         expect = aligned_a and even and not aligned_b and M * N * K * batch >= 1 << 24
-        if M <= 64 and N % 8 == 0 and off_b % 8 == 0 and ldb % 8 == 0:
-            expect = False
         assert ("b_dword" in desc) == expect, (M, N, K, ldb, batch, off_a, off_b, desc)
         if expect:
             taken += 1
-            assert "kernel=tile" in desc and "padded" not in desc, desc
+            # at least 256 tiles of 128 columns fill the GPU by themselves
+            skinny = M <= 64 and N % 8 == 0 and -(-N // 128) * batch < 256
+            assert ("kernel=skinny" if skinny else "kernel=tile") in desc and "padded" not in desc, desc
     assert taken > 60
+    for M, N, K, kw in [(16, 4096, 4096, dict(off_b=2)), (16, 4096, 4096, dict(ldb=4098)), (1, 2048, 8192, dict(ldb=2050, off_b=2)),
+                        (64, 1024, 1024, dict(ldb=1030, batch=3)), (33, 512, 2048, dict(ldb=516))]:
+        desc = _plan(M, N, K, **kw)
+        assert "kernel=skinny_wide " in desc and "b_dword" in desc and "padded" not in desc, desc
+    assert "kernel=tile" in _plan(16, 4090, 4096)                  # N % 8: a piece would cross the row's end
     assert "generic" in _plan(2048, 60, 2048, ws=0)                # without a workspace: as before
     assert "padded" in _plan(1000, 1002, 1004)                     # K % 8: A is copied, and B
     assert "padded=B" in _plan(1000, 1001, 1000)                   # odd rows
@@ -53,6 +58,9 @@ def test_route():
     (200, 196, 1024, 0, 0, 3), (200, 1002, 512, 0, 0, 1), (257, 1030, 520, 6, 0, 1), (128, 2044, 264, 2, 2, 1),
     (300, 500, 72, 4, 6, 2), (70, 4098, 320, 0, 0, 1), (513, 130, 4104, 0, 2, 1), (4090, 4090, 128, 0, 0, 1),
     (64, 70002, 136, 0, 0, 1),
+    # skinny_wide: one to four 16-row blocks, K split and not, streamed once (64 MiB), ragged K, a batch
+    (16, 4096, 4096, 0, 2, 1), (1, 2048, 8192, 2, 0, 1), (33, 8192, 4096, 2, 2, 1), (64, 16392, 264, 4, 6, 1),
+    (48, 1024, 520, 6, 0, 3), (20, 136, 8200, 2, 0, 1), (7, 32000, 128, 2, 2, 1), (16, 128, 8192, 4, 2, 2),
 ])
 def test_results(dtype, M, N, K, gap, off, batch):
     import cmpext3
@@ -82,6 +90,7 @@ def test_results(dtype, M, N, K, gap, off, batch):
 @pytest.mark.parametrize("M,N,K,gap,off,batch", [
     (512, 1001, 1024, 1, 0, 1), (200, 1003, 264, 3, 2, 1), (130, 999, 136, 5, 6, 2), (300, 129, 2048, 1, 0, 1),
     (4095, 4097, 64, 1, 0, 1), (200, 1001, 1024, 7, 0, 1), (512, 1002, 1024, 0, 0, 1), (130, 1004, 136, 2, 2, 2),
+    (16, 1024, 4096, 2, 0, 1), (64, 4096, 1032, 6, 2, 1), (5, 2000, 2056, 0, 2, 3),
 ])
 def test_last_column_of_the_last_row(dtype, M, N, K, gap, off, batch):
     """B's last element, at the very end of the operand (in the middle of a dword where N is
