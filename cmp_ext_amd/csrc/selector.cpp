@@ -690,14 +690,14 @@ int make_plan(const Request& r, Plan* plan) {
     q.b_cols_padded = kn;
     b_bytes = cdiv(rows * cols * 2 * ((batched && r.stride_b != 0) ? r.batch : 1), 256) * 256;
   }
-  if (a_bytes + b_bytes > r.ws_bytes) return st;
   // B as [K, N] whose rows are aligned to 4 bytes (an even N or pitch: images of 14 x 14
   // pixels) needs no copy: a 16-byte LDS-DMA piece only needs a 4-byte aligned source, and
   // the pieces that cross a row's end bring in columns that are not stored (A's would bring
   // in wrong k, hence K % 8 == 0).  MI355X, fp16/bf16, copy + aligned tile -> in place:
   // conv2d [32, 1024, 14, 14] -> 256 25.3 -> 14.7 us, [64, 256, 14, 14] -> 64 15.4 -> 6.8,
   // 512 x 1002 x 2048 34.6 -> 26.5, 64 x 8190 x 4096 64 -> 42, 4096 x 4090 x 4096 140.7 ->
-  // 134.3, 8192 x 3002 x 1024 95.8 -> 91.6: no shape tried was slower.
+  // 134.3, 8192 x 3002 x 1024 95.8 -> 91.6: no shape tried was slower.  Nothing is copied, so
+  // it needs no workspace but a K split's partials.
   if (!pad_a && kn && ab >= 4 && r.ldb % 2 == 0 && (!batched || r.stride_b % 2 == 0) && r.K % 8 == 0) {
     Request d = r;
     d.b_dword = true;
@@ -709,6 +709,7 @@ int make_plan(const Request& r, Plan* plan) {
       return CMPEXT3_OK;
     }
   }
+  if (a_bytes + b_bytes > r.ws_bytes) return st;
   q.align_a = pad_a ? 16 : aa;
   q.align_b = pad_b ? 16 : ab;
   q.align = std::min(std::min(q.align_a, q.align_b), ac);

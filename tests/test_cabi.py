@@ -2,6 +2,7 @@
 include/cmpext3_gemm.h declares, and rejects bad arguments before launching."""
 import ctypes
 import os
+import random
 import re
 
 import pytest
@@ -131,7 +132,10 @@ def _prep(dtype=cabi.F16, layout=cabi.B_KN, M=64, N=64, K=64, A=0x10000, B=0x200
 def test_prepared_call_matches_plan_query():
     for dtype, layout, M, N, K in [(cabi.F16, cabi.B_KN, 4096, 4096, 4096), (cabi.BF16, cabi.B_KN, 4096, 14336, 4096),
                                    (cabi.F16, cabi.B_KN, 16, 8192, 8192), (cabi.F32, cabi.B_KN, 4097, 3001, 2049),
-                                   (cabi.F16, cabi.B_NK, 16, 4096, 14336), (cabi.F32, cabi.B_KN, 16, 8192, 8192)]:
+                                   (cabi.F16, cabi.B_NK, 16, 4096, 14336), (cabi.F32, cabi.B_KN, 16, 8192, 8192),
+                                   # B read in place, with a K split, in two launches
+                                   (cabi.F16, cabi.B_KN, 4096, 4090, 4096), (cabi.BF16, cabi.B_KN, 256, 196, 4096),
+                                   (cabi.F16, cabi.B_KN, 4096, 4100, 4096), (cabi.F16, cabi.B_KN, 4095, 4097, 4096)]:
         st, call = _prep(dtype, layout, M, N, K)
         assert st == cabi.OK
         kid, desc = cabi.describe(call)
@@ -139,6 +143,21 @@ def test_prepared_call_matches_plan_query():
         kid2, desc2 = cabi.plan(dtype, layout, M, N, K, workspace_bytes=need)
         assert (kid, desc) == (kid2, desc2)
         assert need == max(0, cabi.workspace_size(dtype, layout, M, N, K))
+
+
+def test_plans_with_the_queried_workspace():
+    """What the query asks for is enough: the plan with exactly that many bytes is the one
+    without a limit, for products of any size and both layouts."""
+    rng = random.Random(1)
+    size = lambda hi: int(hi ** rng.random())  # noqa: E731
+    for _ in range(3000):
+        dtype, layout, batch = rng.choice([cabi.F16, cabi.BF16, cabi.F32]), rng.choice([0, 1]), rng.choice([1, 1, 1, 2, 8])
+        M, N, K = size(9000), size(15000), size(15000)
+        if rng.random() < 0.5:
+            K = K // 8 * 8 or 8
+        need = cabi.workspace_size(dtype, layout, M, N, K, batch)
+        assert cabi.plan(dtype, layout, M, N, K, batch=batch, workspace_bytes=need) == \
+            cabi.plan(dtype, layout, M, N, K, batch=batch, workspace_bytes=1 << 62), (dtype, layout, M, N, K, batch)
 
 
 def test_prepared_call_limits_workspace():

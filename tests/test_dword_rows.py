@@ -46,7 +46,10 @@ def test_route():
         desc = _plan(M, N, K, **kw)
         assert "kernel=skinny_wide " in desc and "b_dword" in desc and "padded" not in desc, desc
     assert "kernel=tile" in _plan(16, 4090, 4096)                  # N % 8: a piece would cross the row's end
-    assert "generic" in _plan(2048, 60, 2048, ws=0)                # without a workspace: as before
+    for ws in (0, 1 << 20):                                        # nothing is copied: no workspace needed
+        assert "kernel=tile128x128 " in _plan(2048, 60, 2048, ws=ws) and "b_dword" in _plan(2048, 60, 2048, ws=ws)
+        assert "b_dword" in _plan(4096, 4090, 4096, ws=ws)
+    assert "generic" in _plan(2048, 61, 2048, ws=0)                # odd rows: copied, or element by element
     assert "padded" in _plan(1000, 1002, 1004)                     # K % 8: A is copied, and B
     assert "padded=B" in _plan(1000, 1001, 1000)                   # odd rows
     assert "b_dword" not in _plan(1000, 1002, 1000, layout=cabi.B_NK)
@@ -118,3 +121,25 @@ def test_last_column_of_the_last_row(dtype, M, N, K, gap, off, batch):
     # fp32 sums of K products and one rounding to 11 or 8 bits
     bound = K * 2.0 ** -24 * size + 2.0 ** (-11 if dtype == "fp16" else -8) * ref.abs() + 2.0 ** -24
     assert ((out[:, :, N - 9 :].double().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16, 17, 64])
+def test_narrow_strips_without_a_workspace(M):
+    """The narrow skinny kernel on B at an offset of 4 bytes, with a bias per column."""
+    N, K, ldb = 2056, 8200, 2058
+    g = torch.Generator().manual_seed(M)
+    a = (torch.randn((M, K), generator=g) * K ** -0.5).half()
+    b, bias = torch.randn((K, N), generator=g).half(), torch.randn(N, generator=g).half()
+    buf = torch.full((2 + K * ldb + 64,), float("nan"), dtype=torch.half, device="cuda")
+    view = buf[2 : 2 + K * ldb].view(K, ldb)[:, :N]
+    view.copy_(b)
+    c = torch.full((M, N), 3.0, dtype=torch.half, device="cuda")
+    ac, bias_c = a.cuda(), bias.cuda()
+    st, call = cabi.prepare(cabi.F16, cabi.B_KN, ac, K, 0, view.data_ptr(), ldb, 0, c, N, 0, bias_c, M, N, K, 1, 0, 0)
+    assert st == cabi.OK
+    desc = cabi.describe(call)[1]
+    print(M, desc, flush=True)
+    assert "kernel=skinny " in desc and "b_dword" in desc and cabi.call_workspace_size(call) == 0
+    assert cabi.run(call) == cabi.OK
+    assert O.reference_check(c.cpu(), a, b, "fp16", bias) <= O.TOLERANCE["fp16"]

@@ -245,7 +245,7 @@ def test_empty_products_of_every_kernel_plan():
     (cabi.B_KN, 32768, 64, 1024, 1, K_TILE128, 0),    # 256 tiles already fill the GPU
     (cabi.B_KN, 1024, 64, 1024, 32, K_TILE128, 0),    # ... over a batch
     (cabi.B_KN, 2048, 128, 2048, 8, K_TILE128, 0),    # 128 columns: measured slower
-    (cabi.B_KN, 2048, 60, 2048, 1, K_GENERIC, 0),     # [K, N] rows not in 16-byte chunks (no workspace)
+    (cabi.B_KN, 2048, 61, 2048, 1, K_GENERIC, 0),     # [K, N] rows of an odd length (no workspace)
     (cabi.B_NK, 2048, 60, 2048, 1, K_TALL, 32),       # ... which B as [N, K] does not need
 ])
 def test_tall_kernel_for_narrow_b(layout, M, N, K, batch, expect, strip):
