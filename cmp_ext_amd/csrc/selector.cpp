@@ -212,7 +212,12 @@ void split_strips(const Request& r, int64_t splits, Plan* q) {
 // against 29.3).  One block of A: 16, 32 or 48 rows in one round, else 32-row strips two
 // to a CU (x[16, 4096] W[11008, 4096]^T 48 rows 19.9 -> 17.3, W[6144, 4096]^T 32 rows
 // 13.4 -> 10.8; past 48 x 256 rows two of 32 per CU stay ahead: W[14336, 4096]^T 21.3
-// against 22.9 with 64 rows, W[28672, 4096]^T 39.9 against 43.1).
+// against 22.9 with 64 rows, W[28672, 4096]^T 39.9 against 43.1).  Two blocks: at most 80
+// rows, since strips above 64 read each row of W in runs of 256 bytes there and 64-row
+// ones of 512 (three and four blocks: 256 either way); two rounds of 64 rows then stay
+// ahead (x[32, 8192] W[29568, 8192]^T 81.9 against 98.5 us with 128 rows, W[28672, 8192]^T
+// 79.8 against 91.2 with 112, W[24576, 8192]^T 66.7 with 48 against 81.8 with 96; W[20480,
+// 8192]^T 71.9 against 61.7 with 80).
 int skinny_nk_strip(int64_t N, int64_t batch, int mb) {
   if (mb == 1) {
     for (int rows = 16; rows <= 48; rows += 16)
@@ -221,7 +226,7 @@ int skinny_nk_strip(int64_t N, int64_t batch, int mb) {
   }
   int best = 16;
   int64_t least = 0;
-  for (int rows = 16; rows <= 128; rows += 16) {
+  for (int rows = 16; rows <= (mb == 2 ? 80 : 128); rows += 16) {
     const int64_t streamed = cdiv(cdiv(N, rows) * batch, kNumCUs) * (rows + 16 * mb);
     if (rows == 16 || streamed < least) {
       best = rows;

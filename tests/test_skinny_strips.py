@@ -20,7 +20,8 @@ def _strip(M, N, K=4096, batch=1):
 def test_strip_heights():
     for M, N, expect in [(64, 4096, 16), (64, 4104, 32), (64, 8192, 32), (64, 8200, 48), (64, 11008, 48),
                          (64, 12288, 48), (64, 14336, 64), (33, 16384, 64), (33, 17000, 80), (64, 20480, 80),
-                         (64, 24576, 96), (64, 28672, 112), (16, 4096, 16), (16, 4104, 32), (16, 11008, 48),
+                         (64, 24576, 96), (64, 28672, 112), (32, 20480, 80), (32, 24576, 48), (17, 32000, 64),
+                         (16, 4096, 16), (16, 4104, 32), (16, 11008, 48),
                          (1, 12288, 48), (1, 12296, 32), (16, 28672, 32)]:
         assert _strip(M, N) == (expect, False), (M, N)
 
@@ -32,7 +33,7 @@ def test_strips_never_stream_more_than_another_height(M):
     for N in range(4104, 32700, 616):
         rows, split = _strip(M, N)
         if not split:
-            best = min(rounds(N, r) * (r + 16 * mb) for r in range(16, 129, 16))
+            best = min(rounds(N, r) * (r + 16 * mb) for r in range(16, 81 if mb == 2 else 129, 16))
             assert rounds(N, rows) * (rows + 16 * mb) == best, (M, N, rows)
 
 
