@@ -319,8 +319,10 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
 
   // The stages in ring slots slot and slot + 1 (V = u32x4: 32 k), or the one in slot (u32x2:
   // 16 k), on the bf16 instruction: B's next block is read and split among the current
-  // one's products (the fences between blocks only bound the registers; a fixed pattern of
-  // products and vector instructions was no faster).
+  // one's products.  The fences between blocks bound the registers.  128 x 128 tiles of B as
+  // [N,K] take products and vector instructions in a fixed pattern: x[512, 4096] W[4096,
+  // 4096]^T 110 -> 107 us, x[100, 4096] 36.1 -> 34.6; as [K,N] it was slower (4096^3 730 ->
+  // 746), on the small tiles no faster.
   auto split_stages = [&](int slot, auto v) {
     using V = decltype(v);
     using P = F32Planes<V>;
@@ -351,6 +353,12 @@ __device__ __forceinline__ bool f32_tile(const GemmParams& p, unsigned char* sme
       product(small, &P::m, &P::h);
       product(small, &P::h, &P::m);
       product(acc, &P::h, &P::h);
+      if constexpr (PAIR && !KN && BM == 128 && j + 1 < FN) {
+        static_for<6 * FM>([&](auto) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one product,
+          __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // its share of the splitting (52 instructions)
+        });
+      }
       __builtin_amdgcn_sched_barrier(0);
     });
   };
