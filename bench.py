@@ -15,9 +15,10 @@ the first and after the last timed call, so over calls 2..K: the GPU waits from
 the region's first event until the host has enqueued the first call, which is
 host latency, not kernel time; `event_ms_per_step` is the same over all K calls
 from an event before the first), against MI355X's published peaks (dense
-fp16/bf16 MFMA 2516.6 TFLOP/s, fp32 a sixth of it, HBM3E 8 TB/s).  `traffic` (HBM bytes per launch) comes from the committed
-rocprofv3 FETCH_SIZE/WRITE_SIZE summary in profiles/hbm_traffic.json when it
-has an entry for the workload, else null.
+fp16/bf16 MFMA 2516.6 TFLOP/s, fp32 a sixth of it, HBM3E 8 TB/s).  `traffic`
+(HBM bytes per launch) comes from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE
+summary in profiles/hbm_traffic.json when it has an entry for the workload, else
+null.
 
 Inputs: every workload's operands are drawn before any timing starts, by a CPU
 torch.Generator seeded with 0 (A first, then B, in float32, then cast to the

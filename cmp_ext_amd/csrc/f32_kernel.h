@@ -139,7 +139,8 @@ __device__ __forceinline__ void f32_split4(F32Planes<V>& p, int i, f32x4 x) {
 __device__ __forceinline__ f32x4 f32_mma(u32x4 b, u32x4 a, f32x4 c) { return Mfma<__bf16>::mma(b, a, c); }
 __device__ __forceinline__ f32x4 f32_mma(u32x2 b, u32x2 a, f32x4 c) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
-  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, b), __builtin_bit_cast(s16x4, a), c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, b), __builtin_bit_cast(s16x4, a), c, 0,
+                                                   0, 0);
 }
 
 // SPLITK: grid.z = batch * p.splits; this workgroup sums its split's K range and

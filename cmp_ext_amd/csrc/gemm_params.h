@@ -37,16 +37,16 @@ constexpr int kF32ShortK = 16;
 enum KernelId : int {
   kTile256x256 = 0,   // f16/bf16 MFMA 16x16x32, 8 waves of 64x128, LDS-DMA ring
   kTile256x224 = 1,   // same, 8 waves of 64x112 (N tiles of 224)
-  kTile128x128 = 2,   // same, 4 waves of 64x64, two workgroups per CU
+  kTile128x128 = 2,   // same, 4 waves of 64x64, two workgroups per CU, or one with a ring of four K steps
   kSkinny = 3,        // f16/bf16, M <= 64: 32-column strips through an LDS-DMA ring
-  kF32Tile128 = 4,    // fp32 MFMA 16x16x4, 128x128 tile, 4- or 16-byte LDS-DMA ring
+  kF32Tile128 = 4,    // fp32 on the bf16 MFMA (K <= 16: fp32 MFMA 16x16x4), 128x128 tile, 4- or 16-byte LDS-DMA
   kF32Tile64 = 5,     // same, 64x64 tile
   kGeneric16 = 6,     // f16/bf16 any shape and alignment (element loads)
   kSkinnyWide = 7,    // f16/bf16, M <= 64: 128-column strips, K split over workgroups
   kF32Tile96x64 = 8,  // fp32, 96x64 tile
   kTile64x256 = 9,    // f16/bf16 MFMA 16x16x32, 4 waves of 64x64, two workgroups per CU (M <= 64, short K)
-  kSkinnyNK = 10,     // f16/bf16, M <= 64, B is [N,K]: 16- or 32-row strips of W, all of K per workgroup
-  kF32Tile64K4 = 11,  // fp32, 64x64 tile, K split over the workgroup's four waves (few tiles per CU)
+  kSkinnyNK = 10,     // f16/bf16, M <= 64, B is [N,K]: strips of 16 to 128 rows of W, all of K or a K range per workgroup
+  kF32Tile64K4 = 11,  // fp32 MFMA 16x16x4, 64x64 tile, K split over the workgroup's four waves (few tiles per CU)
   kF32Tile16K4 = 12,  // same with 16x64 tiles (M <= 16)
   kStream64x128 = 13, // f16/bf16, M <= 64, K <= 256, B is [K,N]: persistent workgroups stream 128-column tiles
   kStream128x128 = 14,  // same with 128-row tiles (64 < M <= 128)

@@ -51,8 +51,10 @@ double split_cost(const Candidate& c, int64_t M, int64_t N, int64_t K, int64_t b
 
 // Per-area throughput of a CU running the tile, relative to 256x256 (MI355X, fp16
 // 4096^3: 256x256 102.7 us, 128x128 with two workgroups per CU 126.7 us; one 128x128
-// workgroup alone on its CU: 128 x 4096 x 4096 unsplit 41.5 us, 8 x 2048 x 128 x 2048
-// 24.1 us, i.e. 0.61 and 0.53).
+// workgroup alone on its CU with a ring of two K steps: 128 x 4096 x 4096 unsplit 41.5 us,
+// 8 x 2048 x 128 x 2048 24.1 us, i.e. 0.61 and 0.53; with the ring of four that lone tiles
+// of 512 k and more now have (deep_ring) 30.3 us at K = 4096, 0.87, which the choices below
+// do not count on yet).
 const Candidate kTiles16[] = {
     {kTile256x256, 256, 256, 1, 1.00, 1.00},
     {kTile256x224, 256, 224, 1, 0.98, 0.98},
@@ -516,16 +518,17 @@ int make_plan_core(const Request& r, Plan* plan) {
     } else if (tall_ok && r.N <= 64 && r.M >= 1024 && r.K >= 1024 && cdiv(r.M, 128) * r.batch < kNumCUs &&
                (r.K <= 2048 ||
                 (r.K <= 4096 && (r.M * r.batch >= 8192 || (r.layout == kNK && r.N <= 32) || r.N % 4 != 0)))) {
-      // A narrow B (<= 64 columns) under fewer 128-row tiles than CUs: the tile kernels would
-      // split K (or leave CUs idle) to fill the GPU; strips of A's rows over all of K stream
-      // A once instead (MI355X, fp16, best strip vs the selector's tile128x128 (+ split):
-      // 2048 x 64 x 2048 8.5 vs 10.8 us, 8192 x 64 x 2048 10.4 vs 16.1, 16384 x 64 x 2048
-      // 16.6 vs 25.0, 16384 x 16 x 4096 27.7 vs 30.7, attention's P V over 8 x 2048 x 2048
-      // with 64 columns 18.8 vs 25.7; measured slower from K = 8192, with 64 < N <= 128, or
-      // at K = 4096 below 8192 rows -- except B as [N, K] with <= 32 rows, on one or two
-      // 16-row blocks: 4096 x 16 x 4096 7.9 vs 10.8 us, 1024 x 32 x 4096 8.7 vs 9.4 -- or N %
-      // 4 != 0, where a tile cannot split K: 3000 x 33 x 4000 24 vs 51).  64-row strips once they give every CU one and K >=
-      // 2048, else 32-row strips.
+      // A narrow B (<= 64 columns) under fewer 128-row tiles than CUs: the tile kernels
+      // would split K (or leave CUs idle) to fill the GPU; strips of A's rows over all
+      // of K stream A once instead (MI355X, fp16, best strip vs the selector's
+      // tile128x128 (+ split): 2048 x 64 x 2048 8.5 vs 10.8 us, 8192 x 64 x 2048 10.4
+      // vs 16.1, 16384 x 64 x 2048 16.6 vs 25.0, 16384 x 16 x 4096 27.7 vs 30.7,
+      // attention's P V over 8 x 2048 x 2048 with 64 columns 18.8 vs 25.7; measured
+      // slower from K = 8192, with 64 < N <= 128, or at K = 4096 below 8192 rows --
+      // except B as [N, K] with <= 32 rows, on one or two 16-row blocks: 4096 x 16 x
+      // 4096 7.9 vs 10.8 us, 1024 x 32 x 4096 8.7 vs 9.4 -- or N % 4 != 0, where a tile
+      // cannot split K: 3000 x 33 x 4000 24 vs 51).  64-row strips once they give every
+      // CU one and K >= 2048, else 32-row strips.
       p = tall_plan(r, cdiv(r.M, 64) * r.batch >= kNumCUs && r.K >= 2048 ? 64 : 32, p.group_m);
     } else if (tall_ok && r.N <= 64 && r.M >= 1024 && r.K >= 8192 && cdiv(r.M, 32) * r.batch <= 64 &&
                r.N % 4 == 0) {

@@ -10,13 +10,14 @@
 //   * Each wave owns a (BM/WM) x (BN/WN) block of C as 16 x 16 blocks of fp32
 //     accumulators, fed by v_mfma_f32_16x16x32_{f16,bf16}.  The 16-wide block
 //     grain lets a 256 x 224 tile (the MLP shape) use the same grid as 256 x 256.
-//   * Two waves per SIMD: the 256-row tiles run 8 waves (4 x 2, at most 256
-//     VGPRs each) in one workgroup per CU, the 128 x 128 tile 4 waves (2 x 2) in
-//     two workgroups per CU -- or alone on its CU with a deeper ring, when there are
-//     no more workgroups than CUs (deep_ring in tile_inst.h).  One wave's matrix products
-//     then run while the other waits on LDS reads or on the issue of its LDS-DMA loads; measured on
-//     MI355X, 8 waves beat 4 waves of twice the block (fewer fragment bytes per
-//     MFMA, one wave per SIMD) by ~9 % in loop cycles and halve the epilogue.
+//   * Two waves per SIMD: the 256-row tiles run 8 waves (4 x 2, at most 256 VGPRs
+//     each) in one workgroup per CU, the 128 x 128 tile 4 waves (2 x 2) in two
+//     workgroups per CU -- or alone on its CU with a deeper ring, when there are no
+//     more workgroups than CUs (deep_ring in tile_inst.h).  One wave's matrix
+//     products then run while the other waits on LDS reads or on the issue of its
+//     LDS-DMA loads; measured on MI355X, 8 waves beat 4 waves of twice the block
+//     (fewer fragment bytes per MFMA, one wave per SIMD) by ~9 % in loop cycles and
+//     halve the epilogue.
 //   * K steps of BK = 64 go global -> LDS by buffer_load_dwordx4 ... lds (LDS
 //     DMA: no registers, no ds_write) into a ring of two slots (or four).  A step is two
 //     sub-steps of 32 k.  All reads of a step's slot are issued by the end of its

@@ -58,15 +58,16 @@ int cmpext3_matmul_fp16(const void* A, const void* B, void* C, int M, int N, int
 int cmpext3_matmul_bf16(const void* A, const void* B, void* C, int M, int N, int K, void* stream);
 
 /*
- * C[M,N] = A[M,K] * B[K,N] in fp32 (fp32 MFMA, fused multiply-add).
+ * C[M,N] = A[M,K] * B[K,N] in fp32, on the matrix cores with fp32 sums: the fp32
+ * instruction, or the bf16 one with each float as three exact bf16 parts.
  * Replaces launch_matmul_fp32 (src/cuda/fp32_matmul.cu:236-265).
  */
 int cmpext3_matmul_fp32(const float* A, const float* B, float* C, int M, int N, int K, void* stream);
 
 /*
  * Strided row-major forms: C[M,N] = A[M,K] * B[K,N] with row pitches lda >= K,
- * ldb >= N, ldc >= N (elements), fp32 accumulation, output in the input dtype
- * (fp32 MFMA for _f32).  The launchers above with explicit pitches, so a caller
+ * ldb >= N, ldc >= N (elements), fp32 accumulation, output in the input dtype.
+ * The launchers above with explicit pitches, so a caller
  * holding row-pitched views (e.g. a column slice of a larger matrix) needs no
  * copy.  No workspace: M <= 64 products take the unsplit skinny kernel.
  * Replace launch_matmul_fp16/bf16/fp32 (src/cuda/fp16_matmul.cu:301-340,
