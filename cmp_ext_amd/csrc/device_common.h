@@ -98,6 +98,16 @@ __device__ __forceinline__ void dma_load4(i32x4 rsrc, uint32_t voff, uint32_t ld
                : "memory", "m0");
 }
 #pragma clang diagnostic pop
+// Between the steps of a ring that LDS-DMA fills and the whole workgroup reads: at most
+// YOUNGER of this wave's loads are still on their way, its LDS reads are done (not only
+// issued: the compiler may put the products that use them, and its own wait, past the
+// barrier), and so are every other wave's, so the slot just read may be refilled.  Without
+// the wait for the reads another wave's next load could overwrite what this one had yet to
+// fetch, above all the loads past K's end, which return zeros at once.
+template <int YOUNGER>
+__device__ __forceinline__ void ring_fence() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(YOUNGER) : "memory");
+}
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(size_t)(__attribute__((address_space(3))) const void*)p;
 }

@@ -183,15 +183,15 @@ __global__ void __launch_bounds__(256, BM == 16 ? 4 : 2) gemm_f32_kwave_kernel(c
 
   const int steps = (K + BK - 1) / BK;                            // 16-k steps of the workgroup
   const int mine = steps > wave ? (steps - wave + 3) / 4 : 0;     // of this wave
-  // Step j: DMA step j+NS-1 into the slot step j-1 was read from (this wave's own reads
-  // of it completed: their results fed step j-1's MFMAs), compute j, wait for step j+1.
+  // Step j: DMA step j+NS-1 into the slot step j-1 was read from (this wave's own reads of
+  // it are waited for below), compute j, wait for step j+1.
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t) load_step(t);
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NS - 2) * (NA + NB)) : "memory");
   for (int j = 0; j < mine; ++j) {
     load_step(j + NS - 1);
     compute_step(j);
-    asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NS - 2) * (NA + NB)) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"((NS - 2) * (NA + NB)) : "memory");
   }
   asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // no LDS DMA may outlive the loop
 

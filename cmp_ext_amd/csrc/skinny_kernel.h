@@ -166,13 +166,13 @@ __global__ void __launch_bounds__(256) gemm_skinny_narrow_kernel(const GemmParam
   // in LDS and stage st's slot may be refilled.
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t) load_stage(t);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NS - 2) * S::DMA) : "memory");
+  ring_fence<(NS - 2) * S::DMA>();
   for (int st = 0; st < nst; ++st) {
     load_stage(st + NS - 1);
     compute_stage(st);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NS - 2) * S::DMA) : "memory");
+    ring_fence<(NS - 2) * S::DMA>();
   }
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : : : "memory");
+  ring_fence<0>();
 
   // ---- reduce the 4 waves' partial sums through LDS (the ring is free) ----
   // acc[h][mb][r] = C[16*mb + c][n0 + 16*h + 4*g + r]
@@ -383,13 +383,13 @@ __global__ void __launch_bounds__(256) gemm_skinny_nk_kernel(const GemmParams p)
   const int nst = (K + S::KS - 1) / S::KS;
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t) load_stage(t);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NS - 2) * S::DMA) : "memory");
+  ring_fence<(NS - 2) * S::DMA>();
   for (int st = 0; st < nst; ++st) {
     load_stage(st + NS - 1);
     compute_stage(st);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NS - 2) * S::DMA) : "memory");
+    ring_fence<(NS - 2) * S::DMA>();
   }
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : : : "memory");
+  ring_fence<0>();
 
   // ---- reduce the 4 waves' partial sums through LDS (the ring is free) ----
   // acc[h][mb][r] = (X row 16*mb + c) . (W row n0 + 16*h + 4*g + r)

@@ -120,9 +120,9 @@ __global__ void __launch_bounds__(256) gemm_skinny_wide_kernel(const GemmParams 
   // Wait until at most NS-2 younger stages' DMA are in flight, then barrier.
   auto certify = [&]() {
     if (a_cnt == S::A_HI)
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NS - 2) * (S::B_DMA + S::A_HI)) : "memory");
+      ring_fence<(NS - 2) * (S::B_DMA + S::A_HI)>();
     else
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NS - 2) * (S::B_DMA + S::A_LO)) : "memory");
+      ring_fence<(NS - 2) * (S::B_DMA + S::A_LO)>();
   };
 
   // ---- fragments: lane (c = l%16, g = l/16); wave owns columns 32w .. 32w+31 ----
